@@ -6,25 +6,14 @@
 // the reference's batched projections (cpu_decoder.rs:45-62 batch_dot_acc,
 // 398-449; dispatched on the GPU by decoder.rs:3580-4162).
 //
-// Block tile BM x BN (256 x 256, 192 x 256 down to 64 x 64, chosen per
-// shape by a cost model: launch_gemm_f16), K steps of 64, waves in a 2 x WGN grid (WGN = 2:
-// four waves, one per SIMD; WGN = 4: eight, two per SIMD, so one wave's
-// MFMAs run while the other waits), each wave (BM/2) x (BN/WGN) as tiles of
-// v_mfma_f32_32x32x16_f16.  Eight waves measured faster for 256 x 256
-// (16384 x 12288 x 2048: 764-820 against 820-861 us), 192 x 256 and
-// 128 x 128, four for the smaller tiles.  The two largest tiles run a
-// ping-pong schedule of their two wave groups (below); the others run four
-// 16-k slices per K step with the next slice's operand reads issued as one
-// group ahead of the current slice's MFMAs, and the next step's first reads
-// ahead of the last slice's, so no LDS latency is waited for between MFMAs.
-// Both operand tiles go global -> LDS by direct copies (buffer_load ... lds,
-// one 1 KB block per wave instruction) into NS buffers: the copies of K
-// step t+NS are issued as soon as every wave is done with step t's buffers,
-// so NS-1 steps are in flight while another is consumed.  Two stages for
-// the larger tiles (their LDS then still fits two workgroups per CU up to
-// 128 x 128); four for 64 x 64, whose steps are short and latency-bound
-// (420 x 2048 x 6144: 47.8 -> 30 us; three or four stages on the larger
-// tiles cost the second workgroup per CU and measured slower).  LDS row
+// Two kernels of one design, for tiles of 128 x 256 and more (gemm_big_kernel)
+// and down to 64 x 64 (gemm_small_kernel); launch_gemm_f16 chooses per shape by
+// a cost model.  K steps of 64; waves in a 2 x n grid, each computing tiles of
+// v_mfma_f32_32x32x16_f16 as D = B A^T, so that a lane ends with four
+// consecutive columns of a row.  Both operand tiles go global -> LDS by direct
+// copies (buffer_load ... lds, one 1 KB block per wave instruction) into a ring
+// of stages; the copies are inline asm waited for by count, and the barriers
+// are bare, so several steps' copies stay in flight across them.  LDS row
 // layout (both operands): row r is 128 bytes (64 k), its 16-byte chunk c at slot
 // c ^ ((r >> 1) & 7), so an operand read (16 consecutive rows, one chunk)
 // covers 16 distinct 16-byte bank groups.  Rows past M are copied from row
@@ -33,14 +22,19 @@
 // divide by 8, XCD x takes a contiguous run of them and walks them in groups
 // of a few row blocks, so the tiles an XCD runs at one time share a few A
 // and B blocks in its L2.
-// Results are rounded and stored in place; with the residual they go
-// through LDS first, so C is read and written in 8-byte row pieces, all of
-// a row tile's residual reads issued before its first store (one memory
-// round trip per row tile; 256 x 256 at 4269 x 2048 x 2048: 72 against
-// 83.5 us).
+// Every output sums over K in one fixed order whatever the tile.
+// Figures here (us, one MI355X, 28 weight matrices rotated so that they come
+// from HBM, against the two-stage ping-pong and slice-by-slice loops these
+// kernels replace): 4269 x 12288 x 2048 207 -> 189, 4269 x 4096 x 2048 83 -> 68,
+// 4269 x 2048 x 2048 + residual 48 -> 41, 4269 x 2048 x 6144 + residual 138 ->
+// 112, 420 x 12288 x 2048 36.7 -> 31.5, 420 x 4096 x 2048 18.7 -> 15.8,
+// 420 x 2048 x 2048 + residual 10.9 -> 9.6, 131 x 1024 x 3072 + residual 14.5 ->
+// 11.7; weights in the memory-side cache, 420 x 2048 x 6144 + residual 25.7 -> 21.9.
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "kernels.hpp"
 
@@ -48,9 +42,10 @@ namespace qasr {
 
 namespace {
 
-constexpr int kBK = 64;          // k per step
+constexpr int kBK = 64;             // k per step
 constexpr int kRowBytes = kBK * 2;  // 128 bytes of one row per step
-constexpr int kGroupRows = 4;  // row blocks per group of an XCD's tile walk
+constexpr int kSlices = kBK / 16;   // MFMA k-slices per step
+constexpr int kGroupRows = 4;       // row blocks per group of an XCD's tile walk
 
 __device__ __forceinline__ float16v mfma32(const half8v& a, const half8v& b, const float16v& c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
@@ -58,20 +53,305 @@ __device__ __forceinline__ float16v mfma32(const half8v& a, const half8v& b, con
 
 __device__ __forceinline__ int slot_of(int row, int chunk) { return chunk ^ ((row >> 1) & 7); }
 
-// s_waitcnt vmcnt(N) lgkmcnt(0): at most N vector memory operations of this
+// s_waitcnt vmcnt(VM) lgkmcnt(0): at most VM vector memory operations of this
 // wave still in flight, and no LDS operation.
-template <int N>
+template <int VM>
 __device__ __forceinline__ void wait_vm_lgkm0() {
-    static_assert(N >= 0 && N <= 63, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt(0x0070 | (N & 15) | ((N >> 4) << 14));
+    static_assert(VM >= 0 && VM <= 63, "vmcnt range");
+    __builtin_amdgcn_s_waitcnt(0x0070 | (VM & 15) | ((VM >> 4) << 14));
 }
 
-template <int BM, int BN, int NS, bool ACC, int WGN, bool PP>
-__global__ __launch_bounds__(128 * WGN, 1) void gemm_f16_kernel(const f16* __restrict__ A,
-                                                                const f16* __restrict__ B,
-                                                                f16* __restrict__ C, int M, int N,
-                                                                int K) {
-    constexpr int kWaves = 2 * WGN;  // 2 x WGN wave grid
+// A bare workgroup barrier: the caller has waited for what must have landed
+// (a __syncthreads() would also drain the LDS reads still wanted in flight).
+__device__ __forceinline__ void bare_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// dma16 (common.hpp) with the step's byte offset in a scalar register.
+__device__ __forceinline__ void dma16_at(const u32x4v& rsrc, int voff, int soff, uint32_t lds) {
+    asm volatile("buffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voff), "s"(rsrc), "s"(soff), "{m0}"(lds)
+                 : "memory");
+}
+
+// Block coordinates of workgroup bid over nmt row and nnt column blocks (see
+// the XCD note above).
+__device__ __forceinline__ void tile_of(int bid, int nmt, int nnt, int& mt, int& nt) {
+    if (nnt % 8 == 0) {
+        const int x = bid & 7, j = bid >> 3, nper = nnt >> 3;
+        const int grp = j / (kGroupRows * nper);
+        const int gr = min(kGroupRows, nmt - grp * kGroupRows);
+        const int r = j - grp * kGroupRows * nper;
+        mt = grp * kGroupRows + r % gr;
+        nt = x * nper + r / gr;
+    } else {
+        mt = bid % nmt;
+        nt = bid / nmt;
+    }
+}
+
+// The wave's outputs, from D = B A^T tiles: acc[i][j][e] is row m0 + 32 i +
+// l32, column n0 + 32 j + 8 (e / 4) + 4 g + e % 4 (four consecutive columns of
+// a row per lane).  Each 32-row strip goes through the wave's own LDS region
+// `ep` and out as whole row pieces of 16 bytes a lane (without: 2-byte stores,
+// and 256 x 256 x 2048 tiles took ~3 us longer each); with the residual the
+// strip is staged in f32 and all its C pieces are requested before the first
+// use (one memory round trip per strip).  Rows past M are not stored.
+template <int MT, int NT, bool ACC>
+struct Epilogue {
+    static constexpr int kCols = 32 * NT;
+    static constexpr int kRow = ACC ? kCols * 4 + 16 : kCols * 2 + 16;  // padded LDS row, bytes
+    static constexpr int kBytes = 32 * kRow;                            // per wave
+    static constexpr int kPer = kCols / 8;                              // 8-column pieces per row
+    static constexpr int kIt = 32 * kPer / 64;                          // pieces per lane and strip
+
+    static __device__ __forceinline__ void run(float16v (&acc)[MT][NT], char* ep, f16* __restrict__ C, int M,
+                                               int N, int m0, int n0, int lane) {
+        const int g = lane >> 5, l32 = lane & 31;
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            H8 old[ACC ? kIt : 1];
+            if constexpr (ACC) {
+#pragma unroll
+                for (int it = 0; it < kIt; ++it) {
+                    const int p = 64 * it + lane, m = min(m0 + 32 * i + p / kPer, M - 1);
+                    old[it].u = *reinterpret_cast<const uint4*>(C + (int64_t)m * N + n0 + (p % kPer) * 8);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int col = 32 * j + 8 * q + 4 * g;
+                    if constexpr (ACC) {
+                        *reinterpret_cast<float4*>(ep + l32 * kRow + col * 4) =
+                            make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+                    } else {
+                        half4v h;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) h[e] = (f16)acc[i][j][4 * q + e];
+                        *reinterpret_cast<half4v*>(ep + l32 * kRow + col * 2) = h;
+                    }
+                }
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the strip is in LDS
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int it = 0; it < kIt; ++it) {
+                const int p = 64 * it + lane, r = p / kPer, c8 = p % kPer;
+                const int m = m0 + 32 * i + r;
+                H8 o;
+                if constexpr (ACC) {
+                    const float4 lo = *reinterpret_cast<const float4*>(ep + r * kRow + c8 * 32);
+                    const float4 hi = *reinterpret_cast<const float4*>(ep + r * kRow + c8 * 32 + 16);
+                    const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) o.e[e] = (f16)((float)old[it].e[e] + v[e]);
+                } else {
+                    o.u = *reinterpret_cast<const uint4*>(ep + r * kRow + c8 * 16);
+                }
+                if (m < M) *reinterpret_cast<uint4*>(C + (int64_t)m * N + n0 + c8 * 8) = o.u;
+            }
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): reads done before the next strip's writes
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+};
+
+// ---- large tiles -------------------------------------------------------------
+// Four waves in a 2 x 2 grid, one per SIMD, each (BM/2) x (BN/2): the largest
+// wave tile, so the fewest LDS operand bytes per MFMA.  What bounds it is the
+// copies: a CU takes in at most ~85 GB/s of them (a copy-only loop of these
+// tiles), 0.75 us for the 64 KB of a 256 x 256 step against 0.85 us of MFMAs,
+// so they have to run all the time.  With two stages of both operands they
+// could only be issued once a step's reads were done, and had to land before
+// the next step's: 1.4 us a step.  Three stages of A (and of B where LDS holds
+// them; two for 256 columns by 192 or 256 rows, all 160 KB) keep a third of a
+// step or more queued across the barrier: 1.1 us (4269 x 2048 x 6144 with the
+// residual, this tile: 149 -> 118 us).
+//
+// Steps: slice ks + 1's operand reads go out one per MFMA under slice ks's
+// MFMAs.  In slice 3, after MFMA kBar, the wave waits for its copies of step
+// t + 1 and its own reads of step t; past the barrier every wave is done with
+// step t's buffers, so its stage of B and A is refilled (with steps t + NB and
+// t + 3), the copies spread over the MFMAs up to the next barrier: B first, at
+// every second MFMA, then A.
+constexpr int kBar = 2;
+
+template <int BM, int BN, int NB, bool ACC>
+__global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict__ A, const f16* __restrict__ B,
+                                                          f16* __restrict__ C, int M, int N, int K) {
+    constexpr int MT = BM / 64, NT = BN / 64;
+    constexpr int ACOPY = BM / 32, BCOPY = BN / 32;  // copies per wave and step
+    constexpr int S = MT * NT;                       // MFMAs per slice
+    constexpr int NA = 3;
+    constexpr int kABuf = BM * kRowBytes, kBBuf = BN * kRowBytes;
+    static_assert((NB == 2 || NB == 3) && NA * kABuf + NB * kBBuf <= 160 * 1024, "LDS");
+    static_assert(S >= MT + NT && S > kBar, "one operand read per MFMA of a slice");
+    // Position of a copy in MFMAs since the barrier: B copy j at 1 + 2 j, A
+    // copies evenly over the rest, the last before slice 3.
+    constexpr int kPosA0 = 2 * BCOPY + 2, kPosEnd = 4 * S - kBar;
+    constexpr int kStrA = (kPosEnd - kPosA0) / ACOPY;
+    static_assert(kStrA >= 1, "copies fit a step");
+    constexpr int kEarlyB = (S - kBar) / 2 < BCOPY ? (S - kBar) / 2 : BCOPY;  // B copies inside slice 3
+    __shared__ __attribute__((aligned(16))) char smem[NA * kABuf + NB * kBBuf];
+    static_assert(4 * Epilogue<MT, NT, ACC>::kBytes <= NA * kABuf + NB * kBBuf, "epilogue staging fits");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const int g = lane >> 5, l32 = lane & 31;
+    int mt, nt;
+    tile_of(blockIdx.x, (M + BM - 1) / BM, N / BN, mt, nt);
+    const int m0 = mt * BM, n0 = nt * BN;
+
+    const u32x4v ares = make_rsrc_words(A, M * K * 2);
+    const u32x4v bres = make_rsrc_words(B, N * K * 2);
+    // Copy j of wave w fills LDS bytes [(4 j + w) KB, +1 KB) of a stage:
+    // 16-byte unit p = 64 (4 j + w) + lane, row p / 8, slot p % 8.
+    int aoff[ACOPY], boff[BCOPY];
+#pragma unroll
+    for (int j = 0; j < ACOPY; ++j) {
+        const int p = 64 * (4 * j + wave) + lane, row = p >> 3;
+        aoff[j] = min(m0 + row, M - 1) * K * 2 + slot_of(row, p & 7) * 16;
+    }
+#pragma unroll
+    for (int j = 0; j < BCOPY; ++j) {
+        const int p = 64 * (4 * j + wave) + lane, row = p >> 3;
+        boff[j] = (n0 + row) * K * 2 + slot_of(row, p & 7) * 16;
+    }
+    const uint32_t alds = lds_addr(smem) + wave * 1024, blds = alds + NA * kABuf;
+    auto copy_a = [&](int t, int buf, int j) { dma16_at(ares, aoff[j], t * kRowBytes, alds + buf + j * 4096); };
+    auto copy_b = [&](int t, int buf, int j) { dma16_at(bres, boff[j], t * kRowBytes, blds + buf + j * 4096); };
+
+    // Operand addresses of slice ks within a stage (row tile i: + 4 KB i).
+    int ao[kSlices], bo[kSlices];
+#pragma unroll
+    for (int ks = 0; ks < kSlices; ++ks) {
+        const int ra = wm * (BM / 2) + l32, rb = wn * (BN / 2) + l32;
+        ao[ks] = ra * kRowBytes + slot_of(ra, 2 * ks + g) * 16;
+        bo[ks] = NA * kABuf + rb * kRowBytes + slot_of(rb, 2 * ks + g) * 16;
+    }
+    half8v fa[2][MT], fb[2][NT];
+    // Read x of slice ks (a0, b0 .. b(NT-1), a1 ..); after the slice's last its
+    // addresses step, in place, by da and db to the next step's stage (an
+    // address made in a register that MFMAs in flight still read would wait
+    // for them).
+    auto read = [&](int da, int db, int ks, int q, int x) {
+        if (x == 0 || x > NT) {
+            const int i = x == 0 ? 0 : x - NT;
+            fa[q][i] = *(const half8v*)(smem + ao[ks] + i * 4096);
+        } else {
+            fb[q][x - 1] = *(const half8v*)(smem + bo[ks] + (x - 1) * 4096);
+        }
+        if (x == MT + NT - 1) {
+            ao[ks] += da;
+            bo[ks] += db;
+            asm volatile("" : "+v"(ao[ks]), "+v"(bo[ks]));
+        }
+    };
+    float16v acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = (float16v){};
+
+    // Step t.  a0 .. a2, b0 .. b2: stage offsets of steps t, t + 1, t + 2 (NB ==
+    // 2: b2 == b0); the stage of step t - 1 is a2, and b2 or (NB == 2) b1.
+    // F: its copies: bit 0 the rest of B(t - 1 + NB) and bit 1 A(t + 2) under
+    // slices 0..2, bit 2 B(t + NB) after the barrier; bit 3: the last step.
+    auto step = [&](int t, int a0, int a1, int a2, int b0, int b1, int b2, auto Flags) {
+        constexpr int F = decltype(Flags)::value;
+#pragma unroll
+        for (int ks = 0; ks < kSlices; ++ks) {
+#pragma unroll
+            for (int m = 0; m < S; ++m) {
+                const int i = m / NT, j = m % NT, q = ks & 1;
+                acc[i][j] = mfma32(fb[q][j], fa[q][i], acc[i][j]);  // D = B A^T
+                __builtin_amdgcn_sched_barrier(0);
+                if (ks < kSlices - 1) {
+                    if (m < MT + NT) read(a1 - a0, b1 - b0, ks + 1, q ^ 1, m);
+                    const int pos = S - kBar + ks * S + m;
+                    if ((F & 1) && (pos & 1) && pos >= 1 + 2 * kEarlyB && (pos - 1) / 2 < BCOPY)
+                        copy_b(t - 1 + NB, NB == 3 ? b2 : b1, (pos - 1) / 2);
+                    if ((F & 2) && pos >= kPosA0 && (pos - kPosA0) % kStrA == 0 && (pos - kPosA0) / kStrA < ACOPY)
+                        copy_a(t + 2, a2, (pos - kPosA0) / kStrA);
+                } else if (!(F & 8)) {
+                    if (m == kBar) {
+                        wait_vm_lgkm0<F == 7 ? (NB == 2 ? ACOPY : ACOPY + BCOPY) : 0>();
+                        bare_barrier();
+                    }
+                    if (m >= kBar) {
+                        if (m - kBar < MT + NT) read(a2 - a1, b2 - b1, 0, 0, m - kBar);
+                        if (m == S - 1)
+#pragma unroll
+                            for (int x = S - kBar; x < MT + NT; ++x) read(a2 - a1, b2 - b1, 0, 0, x);
+                    }
+                    const int pos = m - kBar;
+                    if ((F & 4) && pos > 0 && (pos & 1) && (pos - 1) / 2 < kEarlyB) copy_b(t + NB, b0, (pos - 1) / 2);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    using Full = std::integral_constant<int, 7>;
+    const int nk = K / kBK;  // >= 3 (gemm_big_fits)
+#pragma unroll
+    for (int j = 0; j < ACOPY; ++j) copy_a(0, 0, j);
+#pragma unroll
+    for (int j = 0; j < BCOPY; ++j) copy_b(0, 0, j);
+#pragma unroll
+    for (int j = 0; j < ACOPY; ++j) copy_a(1, kABuf, j);
+    if constexpr (NB == 3)
+#pragma unroll
+        for (int j = 0; j < BCOPY; ++j) copy_b(1, kBBuf, j);
+#pragma unroll
+    for (int j = 0; j < kEarlyB; ++j) copy_b(NB - 1, (NB - 1) * kBBuf, j);
+    wait_vm_lgkm0<ACOPY + (NB == 3 ? BCOPY : 0) + kEarlyB>();
+    bare_barrier();
+#pragma unroll
+    for (int x = 0; x < MT + NT; ++x) read(kABuf, kBBuf, 0, 0, x);
+    __builtin_amdgcn_sched_barrier(0);
+    int t = 0, a0 = 0, a1 = kABuf, a2 = 2 * kABuf, b0 = 0, b1 = kBBuf, b2 = NB == 3 ? 2 * kBBuf : 0;
+    auto advance = [&]() {
+        const int x = a0, y = b0;
+        a0 = a1;
+        a1 = a2;
+        a2 = x;
+        b0 = b1;
+        b1 = b2;
+        b2 = NB == 3 ? y : b0;
+        ++t;
+    };
+    while (t + NB < nk) {
+        step(t, a0, a1, a2, b0, b1, b2, Full{});
+        advance();
+    }
+    if constexpr (NB == 3) {
+        step(t, a0, a1, a2, b0, b1, b2, std::integral_constant<int, 3>{});
+        advance();
+        step(t, a0, a1, a2, b0, b1, b2, std::integral_constant<int, 0>{});
+    } else {
+        step(t, a0, a1, a2, b0, b1, b2, std::integral_constant<int, 1>{});
+    }
+    advance();
+    step(t, a0, a1, a2, b0, b1, b2, std::integral_constant<int, 8>{});
+    __syncthreads();  // every wave is past its last operand reads
+    Epilogue<MT, NT, ACC>::run(acc, smem + wave * Epilogue<MT, NT, ACC>::kBytes, C, M, N, m0 + wm * (BM / 2),
+                               n0 + wn * (BN / 2), lane);
+}
+
+// ---- small tiles -------------------------------------------------------------
+// Waves in a 2 x WGN grid.  Their K steps are short (a 64 x 64 step is 128
+// MFMA cycles per SIMD against ~380 of LDS traffic), so what counts is that no
+// LDS or memory latency is waited for: a whole step's operands are read into
+// registers under the previous step's MFMAs (one barrier per step, where a
+// read of each 16-k slice under the slice before it waited four LDS latencies:
+// 131 x 1024 x 3072 14.6 -> 11.8 us, 420 x 2048 x 6144 26.2 -> 22.4 us), and
+// NS stages keep NS - 2 steps of copies in flight.
+template <int BM, int BN, int NS, int WGN, bool ACC>
+__global__ __launch_bounds__(128 * WGN, 1) void gemm_small_kernel(const f16* __restrict__ A, const f16* __restrict__ B,
+                                                                  f16* __restrict__ C, int M, int N, int K) {
+    constexpr int kWaves = 2 * WGN;
     constexpr int WM = BM / 2, WN = BN / WGN;
     constexpr int MT = WM / 32, NT = WN / 32;
     static_assert(MT >= 1 && NT >= 1, "wave tile of whole 32 x 32 MFMA tiles");
@@ -79,298 +359,207 @@ __global__ __launch_bounds__(128 * WGN, 1) void gemm_f16_kernel(const f16* __res
     constexpr int BCOPY = BN * kRowBytes / 1024 / kWaves;
     static_assert(ACOPY * kWaves * 1024 == BM * kRowBytes && BCOPY * kWaves * 1024 == BN * kRowBytes,
                   "whole 1 KB copy blocks per wave");
-    // NS stages of both operand buffers in one array: the epilogue reuses all
-    // of it.
-    static_assert(NS >= 2 && NS <= 4, "copy stages");
-    __shared__ __attribute__((aligned(16))) f16 smem[NS * (BM + BN) * kBK];
-    f16(*As)[BM * kBK] = reinterpret_cast<f16(*)[BM * kBK]>(smem);
-    f16(*Bs)[BN * kBK] = reinterpret_cast<f16(*)[BN * kBK]>(smem + NS * BM * kBK);
-
-    // The wave index in a scalar register: the copies' LDS addresses (M0)
-    // are then scalar arithmetic, not a vector add and a readfirstlane each.
+    constexpr int kStepCopies = ACOPY + BCOPY;
+    static_assert(NS >= 2 && NS <= 6 && (NS - 1) * kStepCopies <= 63, "copy stages");
+    constexpr int kABuf = BM * kRowBytes, kBBuf = BN * kRowBytes;
+    __shared__ __attribute__((aligned(16))) char smem[NS * (kABuf + kBBuf)];
+    static_assert(kWaves * Epilogue<MT, NT, ACC>::kBytes <= NS * (kABuf + kBBuf), "epilogue staging fits");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
     const int g = lane >> 5, l32 = lane & 31;
-
-    // Block coordinates (see the XCD note above).
-    const int nmt = (M + BM - 1) / BM, nnt = N / BN;
     int mt, nt;
-    {
-        const int bid = blockIdx.x;
-        if (nnt % 8 == 0 && gridDim.x == (unsigned)(nmt * nnt)) {
-            // XCD x (workgroups x, x + 8, ..) takes column blocks
-            // [x nper, (x+1) nper) and walks them in groups of kGroupRows row
-            // blocks: group after group, each column block of the group's
-            // rows in turn, so the XCD's concurrent tiles share a few A and
-            // B blocks in its L2.
-            const int x = bid & 7, j = bid >> 3, nper = nnt >> 3;
-            const int grp = j / (kGroupRows * nper);
-            const int gr = min(kGroupRows, nmt - grp * kGroupRows);
-            const int r = j - grp * kGroupRows * nper;
-            mt = grp * kGroupRows + r % gr;
-            nt = x * nper + r / gr;
-        } else {
-            mt = bid % nmt;
-            nt = bid / nmt;
-        }
-    }
+    tile_of(blockIdx.x, (M + BM - 1) / BM, N / BN, mt, nt);
     const int m0 = mt * BM, n0 = nt * BN;
 
     const u32x4v ares = make_rsrc_words(A, M * K * 2);
     const u32x4v bres = make_rsrc_words(B, N * K * 2);
-    // This thread's copy sources: instruction j of wave w (of W) fills LDS
-    // bytes [(W j + w) KB, +1 KB): 16-byte unit p = 64 (W j + w) + lane,
-    // row p / 8, slot p % 8, holding chunk slot ^ ((row >> 1) & 7).
-    int aoff[ACOPY], boff[BCOPY];
+    int aoff[ACOPY], boff[BCOPY];  // as in gemm_big_kernel
 #pragma unroll
     for (int j = 0; j < ACOPY; ++j) {
         const int p = 64 * (kWaves * j + wave) + lane, row = p >> 3;
-        const int src = min(m0 + row, M - 1);
-        aoff[j] = src * K * 2 + slot_of(row, p & 7) * 16;
+        aoff[j] = min(m0 + row, M - 1) * K * 2 + slot_of(row, p & 7) * 16;
     }
 #pragma unroll
     for (int j = 0; j < BCOPY; ++j) {
         const int p = 64 * (kWaves * j + wave) + lane, row = p >> 3;
         boff[j] = (n0 + row) * K * 2 + slot_of(row, p & 7) * 16;
     }
+    const uint32_t alds = lds_addr(smem) + wave * 1024, blds = alds + NS * kABuf;
     auto copy_step = [&](int t, int buf) {
         const int kb = t * kRowBytes;
 #pragma unroll
-        for (int j = 0; j < ACOPY; ++j) dma16(ares, aoff[j] + kb, lds_addr(&As[buf][(kWaves * j + wave) * 512]));
+        for (int j = 0; j < ACOPY; ++j) dma16_at(ares, aoff[j], kb, alds + buf * kABuf + j * kWaves * 1024);
 #pragma unroll
-        for (int j = 0; j < BCOPY; ++j) dma16(bres, boff[j] + kb, lds_addr(&Bs[buf][(kWaves * j + wave) * 512]));
+        for (int j = 0; j < BCOPY; ++j) dma16_at(bres, boff[j], kb, blds + buf * kBBuf + j * kWaves * 1024);
     };
-
-    // Operand reads: A tile i (rows wm WM + 32 i + l32) and B tile i (rows
-    // wn WN + 32 i + l32), k-slice ks: chunk 2 ks + g.
-    int arow[MT], brow[NT];
+    int ao[kSlices], bo[kSlices];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) arow[i] = wm * WM + 32 * i + l32;
+    for (int ks = 0; ks < kSlices; ++ks) {
+        const int ra = wm * WM + l32, rb = wn * WN + l32;
+        ao[ks] = ra * kRowBytes + slot_of(ra, 2 * ks + g) * 16;
+        bo[ks] = NS * kABuf + rb * kRowBytes + slot_of(rb, 2 * ks + g) * 16;
+    }
+    half8v fa[2][kSlices][MT], fb[2][kSlices][NT];
+    // The addresses step to the next stage (buf + 1, or back to 0) in place: an
+    // address made in a register the MFMAs in flight still read would wait for
+    // them (420 x 2048 x 6144: 25 against 21.5 us).
+    auto read_step = [&](int buf, int q) {
+        const int da = buf == NS - 1 ? -(NS - 1) * kABuf : kABuf;
+        const int db = buf == NS - 1 ? -(NS - 1) * kBBuf : kBBuf;
 #pragma unroll
-    for (int i = 0; i < NT; ++i) brow[i] = wn * WN + 32 * i + l32;
-
+        for (int ks = 0; ks < kSlices; ++ks) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i) fa[q][ks][i] = *(const half8v*)(smem + ao[ks] + i * 4096);
+#pragma unroll
+            for (int i = 0; i < NT; ++i) fb[q][ks][i] = *(const half8v*)(smem + bo[ks] + i * 4096);
+            ao[ks] += da;
+            bo[ks] += db;
+            asm volatile("" : "+v"(ao[ks]), "+v"(bo[ks]));
+        }
+    };
     float16v acc[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = (float16v){};
-
-    const int nk = K / kBK;
-    constexpr int kStepCopies = ACOPY + BCOPY;
-    static_assert((NS - 1) * kStepCopies <= 63, "vmcnt range");
-    // Wait until at most `pending` steps' copies are in flight (the older
-    // ones have landed), and for every LDS read of this wave.
-    auto wait_steps = [&](int pending) {
-        if (NS > 3 && pending >= 3)
+    auto mfma_step = [&](int q) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < kSlices; ++ks)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[i][j] = mfma32(fb[q][ks][j], fa[q][ks][i], acc[i][j]);  // D = B A^T
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // At most `steps` steps' copies of this wave in flight, no LDS read.
+    auto wait_steps = [&](int steps) {
+        if (NS > 4 && steps >= 4)
+            wait_vm_lgkm0<(NS > 4 ? 4 : 0) * kStepCopies>();
+        else if (NS > 3 && steps >= 3)
             wait_vm_lgkm0<(NS > 3 ? 3 : 0) * kStepCopies>();
-        else if (NS > 2 && pending == 2)
+        else if (NS > 2 && steps >= 2)
             wait_vm_lgkm0<(NS > 2 ? 2 : 0) * kStepCopies>();
-        else if (pending == 1)
+        else if (steps >= 1)
             wait_vm_lgkm0<kStepCopies>();
         else
             wait_vm_lgkm0<0>();
     };
+    const int nk = K / kBK;
     const int npro = nk < NS ? nk : NS;  // steps copied ahead
     for (int t = 0; t < npro; ++t) copy_step(t, t);
-    wait_steps(npro - 1);
-    __syncthreads();
-
-    // Operand registers of two k-slices: slice ks+1's reads are issued as
-    // one group ahead of slice ks's MFMAs, so their LDS latency runs under
-    // those MFMAs; sched_barrier keeps the compiler from moving a read next
-    // to its first use.
-    half8v a[2][MT], b[2][NT];
-    auto read_slice = [&](const f16* as, const f16* bs, int ks, int q) {
+    wait_steps(npro - 1 < 4 ? npro - 1 : 4);
+    bare_barrier();
+    read_step(0, 0);
+    // Step t (stage buf, operands in registers q): its reads and the copies of
+    // step t + 1 have landed in every wave, so stage buf takes step t + NS and
+    // step t + 1 is read under this step's MFMAs.
+    auto next = [&](int b) { return b + 1 == NS ? 0 : b + 1; };
+    int t = 0, buf = 0;
+    for (; t + 1 + NS < nk; t += 2) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
-            a[q][i] = *(const half8v*)&as[arow[i] * kBK + slot_of(arow[i], 2 * ks + g) * 8];
-#pragma unroll
-        for (int i = 0; i < NT; ++i)
-            b[q][i] = *(const half8v*)&bs[brow[i] * kBK + slot_of(brow[i], 2 * ks + g) * 8];
-    };
-    auto mfma_slice = [&](int q) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int j = 0; j < NT; ++j) acc[i][j] = mfma32(a[q][i], b[q][j], acc[i][j]);
-    };
-    constexpr int kSlices = kBK / 16;
-    static_assert(kSlices == 4, "slices 0..2 then the step boundary under slice 3");
-    // K step t from buffer t % NS.  All but the last step end with the step
-    // boundary (straight-line code, so the compiler's waits track exactly
-    // which reads are outstanding).
-    auto k_step = [&](int t, bool last) {
-        const int buf = t % NS;
-        const f16* as = As[buf];
-        const f16* bs = Bs[buf];
-        // Slice 0's reads were issued under the previous step's last MFMAs:
-        // done by now.  Waiting here explicitly keeps the compiler from
-        // waiting for the reads issued next, which it would otherwise
-        // assume pending across the loop edge.
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-#pragma unroll
-        for (int ks = 0; ks + 1 < kSlices; ++ks) {
-            read_slice(as, bs, ks + 1, (ks + 1) & 1);
-            __builtin_amdgcn_sched_barrier(0);
-            mfma_slice(ks & 1);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int u = 0; u < 2; ++u) {
+            wait_vm_lgkm0<(NS - 2) * kStepCopies>();
+            bare_barrier();
+            copy_step(t + u + NS, buf);
+            buf = next(buf);
+            read_step(buf, u ^ 1);
+            mfma_step(u);
         }
-        // Slice 3's operands are in registers.  Once every wave has them
-        // (all of its LDS reads of this buffer returned) and step t+1's
-        // copies have landed (those of the steps after it may still fly),
-        // refill this buffer with step t+NS and read step t+1's slice 0,
-        // both under slice 3's MFMAs.
-        if (!last) {
-            const int newest = t + NS - 1 < nk - 1 ? t + NS - 1 : nk - 1;  // last step copied
-            wait_steps(newest - (t + 1));
-            __syncthreads();
-            if (t + NS < nk) copy_step(t + NS, buf);
-            const int nb = (t + 1) % NS;
-            read_slice(As[nb], Bs[nb], 0, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        mfma_slice(1);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    if constexpr (PP) {
-        // Ping-pong (the 256 x 256 and 192 x 256 tiles): waves 0-3 (group 0)
-        // and 4-7 (group 1), one of each per SIMD, alternate strictly between
-        // a read phase (a K step's operands, LDS -> registers, and the copies
-        // of the next step) and an MFMA phase (the step's 32 or 24 MFMAs),
-        // group 1 one phase behind, every phase ending at a workgroup
-        // barrier: while one wave of a SIMD reads, the other feeds the matrix
-        // core.  16384 x 12288 x 2048, same box: 256 x 256 714-722 us
-        // against 787-795 with group 1's copies moved as described below,
-        // and ~800 with the pipelined loop; 192 x 256 801-805 against
-        // 827-831.  Half-step phases (twice the barriers) measured in
-        // between; 128 x 128 with them (four MFMAs a phase) was slower than
-        // its pipelined loop.  Step t is read in global phase 2t by group 0
-        // and 2t + 1 by group 1 and multiplied one phase later.  At its read
-        // of step t (t >= 1) a wave copies its share of step t + 1 into
-        // buffer (t + 1) % 2, which both groups finished reading (step t - 1)
-        // in phases 2t - 2 and 2t - 1; step t + 1 is read from phase 2t + 2
-        // on, and every wave waits for its own copies (vmcnt) before the
-        // barrier that ends phase 2t + 1.  Group 1 thus waits in the phase it
-        // copies in; moving its copies into its MFMA phase one step earlier,
-        // so that they have two phases, measured 11% slower (the copy
-        // instructions then hold up the MFMA issue).  The K order of every
-        // output is that of the other tiles, so the bits are too.
-        static_assert(NS == 2 && kWaves == 8, "ping-pong: two stages, two waves per SIMD");
-        const int grp = __builtin_amdgcn_readfirstlane(wave >> 2);
-        half8v pa[kSlices][MT], pb[kSlices][NT];
-        // The one-phase offset is a barrier that only group 1 executes at the
-        // start and only group 0 at the end.  The condition is uniform per
-        // wave (readfirstlane), and every wave executes 2 nk + 1 barriers in
-        // all, so each hardware barrier still gathers all eight waves: the
-        // k-th barrier of a group-0 wave meets the k-th of a group-1 wave.
-        if (grp == 1) __syncthreads();
-        for (int t = 0; t < nk; ++t) {
-            if (t >= 1 && t + 1 < nk) copy_step(t + 1, (t + 1) & 1);
-            const f16* as = As[t & 1];
-            const f16* bs = Bs[t & 1];
+    }
+    for (; t < nk; t += 2) {
 #pragma unroll
-            for (int ks = 0; ks < kSlices; ++ks) {
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-                    pa[ks][i] = *(const half8v*)&as[arow[i] * kBK + slot_of(arow[i], 2 * ks + g) * 8];
-#pragma unroll
-                for (int i = 0; i < NT; ++i)
-                    pb[ks][i] = *(const half8v*)&bs[brow[i] * kBK + slot_of(brow[i], 2 * ks + g) * 8];
+        for (int u = 0; u < 2; ++u) {
+            if (t + u < nk) {
+                const int newest = min(t + u + NS - 1, nk - 1);  // last step copied
+                wait_steps(newest - (t + u + 1));
+                bare_barrier();
+                if (t + u + NS < nk) copy_step(t + u + NS, buf);
+                buf = next(buf);
+                if (t + u + 1 < nk) read_step(buf, u ^ 1);
+                mfma_step(u);
             }
-            if (grp == 1) wait_vm_lgkm0<0>();
-            __syncthreads();  // (lgkmcnt(0): this phase's reads are in registers)
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int ks = 0; ks < kSlices; ++ks)
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) acc[i][j] = mfma32(pa[ks][i], pb[ks][j], acc[i][j]);
-            __builtin_amdgcn_sched_barrier(0);
-            if (grp == 0) wait_vm_lgkm0<0>();
-            __syncthreads();
         }
-        if (grp == 0) __syncthreads();
-    } else {
-        read_slice(As[0], Bs[0], 0, 0);
-        for (int t = 0; t + 1 < nk; ++t) k_step(t, false);
-        k_step(nk - 1, true);
     }
-
-    // acc[i][j][e]: row wm WM + 32 i + 8 (e / 4) + 4 g + e % 4, column
-    // wn WN + 32 j + l32 of the block.
-    if constexpr (!ACC) {
-        // Plain result: each value rounded and stored where it sits (the
-        // stores need no wait, and measured faster than staging them).
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int m = m0 + wm * WM + 32 * i + 8 * (e >> 2) + 4 * g + (e & 3);
-                if (m >= M) continue;
-                f16* crow = C + (int64_t)m * N + n0 + wn * WN + l32;
-#pragma unroll
-                for (int j = 0; j < NT; ++j) crow[32 * j] = (f16)acc[i][j][e];
-            }
-        return;
-    }
-    // With the residual: row tile i of the wave (32 rows x WN columns) goes
-    // through this wave's LDS region as f32 (rows padded so the two lane
-    // halves' writes fall on different banks), then out as row-contiguous
-    // 4-column pieces: one 8-byte load of C and one 8-byte store per piece,
-    // instead of a dependent 2-byte load per value.
-    __syncthreads();  // every wave is past its last operand reads
-    constexpr int EP = WN + 8;      // padded row, floats
-    constexpr int CPR = WN / 4;     // 4-column pieces per row
-    constexpr int RPP = 64 / CPR;   // rows per pass of the wave
-    static_assert(kWaves * 32 * EP * 4 <= NS * (BM + BN) * kBK * 2, "epilogue staging fits the operand buffers");
-    float* ep = reinterpret_cast<float*>(smem) + wave * (32 * EP);
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) ep[(8 * (e >> 2) + 4 * g + (e & 3)) * EP + 32 * j + l32] = acc[i][j][e];
-        // Every residual piece of the row tile is requested before the first
-        // store (rows past M read row M - 1 and are not stored), so the
-        // tile waits for one memory round trip, not one per piece.
-        constexpr int kIt = 32 / RPP;
-        half4v old[kIt];
-#pragma unroll
-        for (int it = 0; it < kIt; ++it) {
-            const int rr = it * RPP + lane / CPR, cc = (lane % CPR) * 4;
-            const int m = min(m0 + wm * WM + 32 * i + rr, M - 1);
-            old[it] = *reinterpret_cast<const half4v*>(C + (int64_t)m * N + n0 + wn * WN + cc);
-        }
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int it = 0; it < kIt; ++it) {
-            const int rr = it * RPP + lane / CPR, cc = (lane % CPR) * 4;
-            const float4 v = *(const float4*)&ep[rr * EP + cc];
-            const int m = m0 + wm * WM + 32 * i + rr;
-            if (m >= M) continue;
-            half4v o;
-            o[0] = (f16)((float)old[it][0] + v.x);
-            o[1] = (f16)((float)old[it][1] + v.y);
-            o[2] = (f16)((float)old[it][2] + v.z);
-            o[3] = (f16)((float)old[it][3] + v.w);
-            *reinterpret_cast<half4v*>(C + (int64_t)m * N + n0 + wn * WN + cc) = o;
-        }
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): reads done before the next tile's writes
-        __builtin_amdgcn_wave_barrier();
-    }
+    // Every wave's last operand reads returned before the last step's barrier.
+    Epilogue<MT, NT, ACC>::run(acc, smem + wave * Epilogue<MT, NT, ACC>::kBytes, C, M, N, m0 + wm * WM, n0 + wn * WN,
+                               lane);
 }
 
-template <int BM, int BN, int NS = 2, int WGN = 2, bool PP = false>
-hipError_t launch_shape(const f16* A, const f16* B, f16* C, int M, int N, int K, bool accumulate,
-                        hipStream_t stream) {
-    const dim3 grid((unsigned)(((M + BM - 1) / BM) * (N / BN)));
-    if (accumulate)
-        hipLaunchKernelGGL((gemm_f16_kernel<BM, BN, NS, true, WGN, PP>), grid, dim3(128 * WGN), 0, stream, A, B, C, M, N, K);
+struct GemmCall {
+    const f16* A;
+    const f16* B;
+    f16* C;
+    int M, N, K;
+    bool accumulate;
+    hipStream_t stream;
+};
+
+template <int BM, int BN, int NB>
+hipError_t launch_big(const GemmCall& c) {
+    const dim3 grid((unsigned)(((c.M + BM - 1) / BM) * (c.N / BN)));
+    if (c.accumulate)
+        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, true>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     else
-        hipLaunchKernelGGL((gemm_f16_kernel<BM, BN, NS, false, WGN, PP>), grid, dim3(128 * WGN), 0, stream, A, B, C, M, N, K);
+        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, false>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     return hipGetLastError();
+}
+
+template <int BM, int BN, int NS, int WGN>
+hipError_t launch_small(const GemmCall& c) {
+    const dim3 grid((unsigned)(((c.M + BM - 1) / BM) * (c.N / BN)));
+    if (c.accumulate)
+        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, true>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+    else
+        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, false>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+    return hipGetLastError();
+}
+
+// Block tiles.  `occ` workgroups of a tile fit a CU (LDS).  A workgroup takes
+// fix + (K / 64) step us: the large tiles, alone on a CU, run in whole rounds
+// of one per CU; the small ones take step[0] alone and step[1] two to a CU
+// (in between, as the square root of the share of CUs with two), and fill in
+// behind each other, so a last part round costs little more than its share.
+// The figures are sweeps of every tile over the 1.7B and 0.6B projections at 64
+// to 4,269 rows and a 16384 x 12288 x 2048 product, weights coming from HBM.
+struct Tile {
+    int bm, bn, occ;
+    float fix, step[2];
+    int min_steps;  // K steps the kernel needs
+    hipError_t (*launch)(const GemmCall&);
+};
+const Tile kTiles[] = {{256, 256, 1, 6.5f, {1.50f, 0.0f}, 2, launch_big<256, 256, 2>},
+                       {192, 256, 1, 6.0f, {1.10f, 0.0f}, 2, launch_big<192, 256, 2>},
+                       {128, 256, 1, 5.5f, {0.82f, 0.0f}, 3, launch_big<128, 256, 3>},
+                       {64, 128, 2, 4.0f, {0.40f, 0.62f}, 1, launch_small<64, 128, 3, 2>},
+                       {128, 64, 2, 4.0f, {0.38f, 0.62f}, 1, launch_small<128, 64, 3, 2>},
+                       {64, 64, 2, 3.5f, {0.25f, 0.44f}, 1, launch_small<64, 64, 4, 2>}};
+constexpr int kNumTiles = (int)(sizeof kTiles / sizeof kTiles[0]);
+constexpr float kSecondLaunchUs = 2.0f;
+
+float tile_us(const Tile& c, int64_t rows, int N, int K, int64_t cus) {
+    const int64_t tiles = (rows + c.bm - 1) / c.bm * (N / c.bn);
+    const float steps = (float)(K / kBK);
+    if (c.occ == 1) return (float)((tiles + cus - 1) / cus) * (c.fix + steps * c.step[0]);
+    const float per_cu = (float)tiles / (float)cus;
+    if (per_cu <= 1.0f) return c.fix + steps * c.step[0];
+    if (per_cu <= 2.0f) return c.fix + steps * (c.step[0] + (c.step[1] - c.step[0]) * std::sqrt(per_cu - 1.0f));
+    const float rounds = 0.5f * per_cu;
+    return (rounds + 0.5f * (std::ceil(rounds) - rounds)) * (c.fix + steps * c.step[1]);
+}
+
+// The tile of least predicted time for `rows` rows.
+const Tile& best_tile(int64_t rows, int N, int K, int64_t cus, float* us) {
+    const Tile* best = nullptr;
+    for (const Tile& c : kTiles) {
+        if (K / kBK < c.min_steps) continue;
+        const float t = tile_us(c, rows, N, K, cus);
+        if (!best || t < *us) {
+            best = &c;
+            *us = t;
+        }
+    }
+    return *best;
 }
 
 }  // namespace
@@ -383,53 +572,46 @@ bool gemm_f16_fits(int M, int N, int K) {
 hipError_t launch_gemm_f16(const f16* A, const f16* B, f16* C, int M, int N, int K, bool accumulate,
                            int cus, hipStream_t stream) {
     if (!gemm_f16_fits(M, N, K)) return hipErrorInvalidValue;
-    // Block tile: the one with the least predicted time.  A candidate fits
-    // `occ` workgroups per CU (LDS); its tiles run in rounds of occ x cus,
-    // with c = min(occ, ceil(tiles / cus)) of them sharing a CU, and a round
-    // takes c x tile area x cost[c - 1], the measured time per unit area of
-    // one of c workgroups sharing a CU (small tiles alone on a CU wait on
-    // their latencies; a second or third one on the CU hides them).  The
-    // costs (256 x 256 = 52) come from sweeps of every candidate over the
-    // 1.7B projections at 420 and 4,269 rows and a 16384 x 12288 x 2048
-    // product; at each the model picks the fastest tile or one within about
-    // 12% of it.  (192 x 256 is for N = 2048 at a few thousand rows: 4,269
-    // rows make 184 such tiles, one round, against 136 of 256 x 256.)
-    // Every tile accumulates each output over K in the same order, so the
-    // choice never changes a result's bits.
-    // QASR_GEMM_TILE = 1..6 forces candidate 1..6 (the tests compare them).
-    struct Cand { int bm, bn, occ; float cost[3]; };
-    constexpr Cand cands[] = {{256, 256, 1, {52.0f, 0.0f, 0.0f}},      // 8 waves, ping-pong
-                              {192, 256, 1, {57.0f, 0.0f, 0.0f}},      // 8 waves, ping-pong
-                              {128, 128, 2, {72.0f, 60.0f, 0.0f}},     // 8 waves
-                              {64, 128, 3, {125.0f, 105.0f, 85.0f}},   // 4 waves
-                              {128, 64, 3, {125.0f, 105.0f, 85.0f}},   // 4 waves
-                              {64, 64, 2, {170.0f, 112.0f, 0.0f}}};    // 4 waves, 4 stages
-    constexpr int kCands = (int)(sizeof cands / sizeof cands[0]);
     const int64_t ncu = std::max(1, cus);
-    int best = 0;
-    double best_t = 0.0;
-    for (int i = 0; i < kCands; ++i) {
-        const Cand& c = cands[i];
-        const int64_t tiles = (int64_t)((M + c.bm - 1) / c.bm) * (N / c.bn);
-        const int64_t rounds = (tiles + c.occ * ncu - 1) / (c.occ * ncu);
-        const int conc = (int)std::min<int64_t>(c.occ, (tiles + ncu - 1) / ncu);
-        const double t = (double)rounds * conc * c.bm * c.bn * c.cost[conc - 1];
-        if (i == 0 || t < best_t) {
-            best = i;
-            best_t = t;
-        }
-    }
+    GemmCall c{A, B, C, M, N, K, accumulate, stream};
+    // QASR_GEMM_TILE = 1..6 forces that tile for all rows (the tests compare
+    // them; one whose kernel needs more K steps than there are is not forced).
     const char* forced = std::getenv("QASR_GEMM_TILE");
     const int f = forced ? std::atoi(forced) : 0;
-    if (f >= 1 && f <= kCands) best = f - 1;
-    switch (best) {
-        case 0: return launch_shape<256, 256, 2, 4, true>(A, B, C, M, N, K, accumulate, stream);
-        case 1: return launch_shape<192, 256, 2, 4, true>(A, B, C, M, N, K, accumulate, stream);
-        case 2: return launch_shape<128, 128, 2, 4>(A, B, C, M, N, K, accumulate, stream);
-        case 3: return launch_shape<64, 128, 2, 2>(A, B, C, M, N, K, accumulate, stream);
-        case 4: return launch_shape<128, 64, 2, 2>(A, B, C, M, N, K, accumulate, stream);
-        default: return launch_shape<64, 64, 4, 2>(A, B, C, M, N, K, accumulate, stream);
+    if (f >= 1 && f <= kNumTiles && K / kBK >= kTiles[f - 1].min_steps) return kTiles[f - 1].launch(c);
+    // One tile for all rows, or a tile's whole rounds for the first rows and a
+    // second launch with the best tile for the rest, whichever the model calls
+    // fastest: 4,269 rows of gate|up are 816 tiles of 256 x 256, 3.2 rounds
+    // that take four (199 us); three full rounds over 4,096 rows and small
+    // tiles for the other 173 take 189.  Every tile sums each output
+    // over K in the same order, so the choice never changes a bit.
+    float best_us = 0.0f;
+    const Tile* t1 = &best_tile(M, N, K, ncu, &best_us);
+    const Tile* t2 = nullptr;
+    int m1 = M;
+    for (const Tile& c1 : kTiles) {
+        if (K / kBK < c1.min_steps) continue;
+        const int64_t per_row = N / c1.bn, full = (int64_t)c1.occ * ncu;
+        const int64_t rounds = (M / c1.bm) * per_row / full;
+        const int64_t rows = rounds * full / per_row * c1.bm;
+        if (rows <= 0 || rows >= M) continue;
+        float rest = 0.0f;
+        const Tile& c2 = best_tile(M - rows, N, K, ncu, &rest);
+        const float t = tile_us(c1, rows, N, K, ncu) + rest + kSecondLaunchUs;
+        if (t < best_us) {
+            best_us = t;
+            t1 = &c1;
+            t2 = &c2;
+            m1 = (int)rows;
+        }
     }
+    c.M = m1;
+    const hipError_t e = t1->launch(c);
+    if (e != hipSuccess || !t2) return e;
+    c.A = A + (int64_t)m1 * K;
+    c.C = C + (int64_t)m1 * N;
+    c.M = M - m1;
+    return t2->launch(c);
 }
 
 }  // namespace qasr

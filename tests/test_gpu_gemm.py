@@ -138,3 +138,49 @@ def test_gemm_tile_choice_keeps_bits(gpu, m, n, k, accumulate, monkeypatch):
     ref = ref.cpu().numpy().astype(np.float64)
     bound = 0.5 * _f16_spacing(ref) + 2 * (k + 1) * 2.0 ** -24 * mag.cpu().numpy()
     assert np.all(np.abs(outs[0].astype(np.float64) - ref) <= bound)
+
+
+# Edges of the two kernels' loops and of the row split: K steps around the
+# large tiles' copy stages (2 .. 7, odd ones among them), one row more and less
+# than a block, and a row count that takes a second launch for its last rows.
+EDGES = [(255, 256, 192), (257, 256, 256), (129, 512, 320), (385, 768, 448), (1, 256, 384),
+         (4096 + 37, 4096, 256), (513, 12288, 128)]
+
+
+@pytest.mark.parametrize("m,n,k", EDGES)
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_gemm_loop_edges_every_tile(gpu, m, n, k, accumulate, monkeypatch):
+    """At each edge shape every tile gives one set of bits, rows of the call
+    alone give the same bits as inside it, and they meet the fp32 bound."""
+    import torch
+
+    import qasr_attn
+    from gpu_helpers import say
+
+    g = torch.Generator(device="cuda").manual_seed(7300 + m + n + k + int(accumulate))
+    a = torch.randn((m, k), generator=g, device="cuda").to(torch.float16)
+    b = (torch.randn((n, k), generator=g, device="cuda") * 0.05).to(torch.float16)
+    c0 = torch.randn((m, n), generator=g, device="cuda").to(torch.float16)
+    want = None
+    for tile in [0] + TILES:
+        if tile:
+            monkeypatch.setenv("QASR_GEMM_TILE", str(tile))
+        else:
+            monkeypatch.delenv("QASR_GEMM_TILE", raising=False)
+        say(f"gemm {m}x{n}x{k} accumulate={accumulate} tile {tile}")
+        c = c0.clone()
+        qasr_attn.gemm_f16(g_ctx(), a, b, c, accumulate=accumulate)
+        want = c if want is None else want
+        assert torch.equal(c.view(torch.int16), want.view(torch.int16)), tile
+    monkeypatch.delenv("QASR_GEMM_TILE", raising=False)
+    r0 = max(0, m - 40)
+    tail = c0[r0:].clone()
+    qasr_attn.gemm_f16(g_ctx(), a[r0:].contiguous(), b, tail, accumulate=accumulate)
+    assert torch.equal(tail.view(torch.int16), want[r0:].view(torch.int16))
+    bt = b.float().t().contiguous()
+    ref, mag = torch.mm(a.float(), bt), torch.mm(a.float().abs(), bt.abs())
+    if accumulate:
+        ref, mag = ref + c0.float(), mag + c0.float().abs()
+    ref = ref.cpu().numpy()
+    bound = 0.5 * _f16_spacing(ref) + 2 * (k + 1) * 2.0 ** -24 * mag.cpu().numpy()
+    assert np.all(np.abs(want.cpu().numpy().astype(np.float64) - ref) <= bound)
