@@ -392,6 +392,38 @@ def test_int8_projections_equal_dequantized_f16(gpu, model, batch, blas, monkeyp
     assert np.array_equal(runs[0][1], runs[1][1])
 
 
+@pytest.mark.parametrize("hs,inter,int8", [(1024, 3072, ("o_proj", "down_proj")),
+                                            (256, 640, PROJECTIONS),
+                                            (320, 384, ("gate_proj", "up_proj")),
+                                            (256, 136, ("q_proj", "k_proj", "v_proj", "down_proj"))])
+def test_prefill_dequantises_any_set_of_projections(gpu, hs, inter, int8):
+    """A layer's int8 matrices are dequantised in one launch: any subset of
+    them, sizes that leave part of a workgroup, layers that differ; prefill
+    logits and tokens equal those over host-dequantised weights, bitwise."""
+    import torch
+
+    from gpu_helpers import say
+
+    cfg = dict(CFG_0P6B, hs=hs, inter=inter, layers=3, vocab=4096)
+    W = synth_weights(cfg, SEED_BASE + 1300 + hs + inter, device="cuda")
+    W8, Wdq = dict(W), dict(W)
+    for key in list(W):
+        if isinstance(key, tuple) and key[1] in int8 and key[0] != 1:  # layer 1 stays f16
+            q, s = _quantize_rows(W[key])
+            W8[key], W8[(key[0], key[1] + "_scale")] = q, s
+            Wdq[key] = (q.float() * s[:, None]).half()
+    out = []
+    for label, weights in (("int8", W8), ("f16", Wdq)):
+        say(f"hs {hs} inter {inter} int8 {int8}: prefill over {label} weights")
+        dec = _native(cfg, weights, 1, 1024, max_rows=64)
+        lg = torch.empty((cfg["vocab"],), dtype=torch.float32, device="cuda")
+        tok = dec.prefill(_prompt(SEED_BASE + 1310, 45, hs), 0, logits=lg)
+        out.append((tok, lg.cpu().numpy().copy()))
+        dec.close()
+    assert out[0][0] == out[1][0]
+    assert np.array_equal(out[0][1], out[1][1])
+
+
 @pytest.mark.parametrize("model,batch,int8,lds", [("1.7B", 16, False, "1"), ("0.6B", 1, False, "1"),
                                                   ("0.6B", 3, False, "1"), ("1.7B", 2, False, "1"),
                                                   ("1.7B", 16, True, "1"), ("0.6B", 5, True, "1"),
