@@ -22,6 +22,21 @@ __device__ __forceinline__ float h2f(f16 h) { return (float)h; }
 // subnormals kept -- the rounding of half::f16::from_f32.
 __device__ __forceinline__ f16 f2h(float f) { return (f16)f; }
 
+// f16(x) of an f32 value that is first rounded to f32: the reference's
+// f16::from_f32 of an f32 result.  Without the register barrier the compiler
+// folds the product or fma producing x into v_fma_mixlo_f16, which rounds the
+// exact result once, straight to f16, and differs from f16(f32(.)) on about
+// 2 in 10^5 products (measured on gfx950).
+__device__ __forceinline__ f16 f16_of_f32(float x) {
+    asm volatile("" : "+v"(x));
+    return (f16)x;
+}
+
+// SiLU(g) * u in f32 (silu, cpu_decoder.rs): g / (1 + e^-g), then times u.
+__device__ __forceinline__ float silu_times(float g, float u) {
+    return g / (1.0f + expf(-g)) * u;
+}
+
 // 16 bytes = 8 halves, moved as one dwordx4.
 union H8 {
     uint4 u;

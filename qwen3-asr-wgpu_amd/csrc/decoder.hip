@@ -39,7 +39,9 @@
 #include "common.hpp"
 
 using qasr::f16;
+using qasr::f16_of_f32;
 using qasr::H8;
+using qasr::silu_times;
 using qasr_abi::DeviceScope;
 using qasr_abi::fail;
 using qasr_abi::hip_fail;
@@ -183,21 +185,6 @@ __global__ __launch_bounds__(kNormThreads) void rms_norm_kernel(const f16* __res
 
 // h[r][i] = f16(g / (1 + exp(-g)) * u), g|u = gu[r][i], gu[r][inter + i]
 // (cpu_decoder.rs:442-448).  8 elements per thread.
-// f16(x) of an f32 value that is first rounded to f32: the reference's
-// f16::from_f32 of an f32 result.  Without the register barrier the compiler
-// folds the product or fma producing x into v_fma_mixlo_f16, which rounds the
-// exact result once, straight to f16, and differs from f16(f32(.)) on about
-// 2 in 10^5 products (measured on gfx950).
-__device__ __forceinline__ f16 f16_of_f32(float x) {
-    asm volatile("" : "+v"(x));
-    return (f16)x;
-}
-
-// SiLU(g) * u in f32 (silu, cpu_decoder.rs): g / (1 + e^-g), then times u.
-__device__ __forceinline__ float silu_times(float g, float u) {
-    return g / (1.0f + expf(-g)) * u;
-}
-
 __global__ __launch_bounds__(256) void silu_mul_kernel(const f16* __restrict__ gu, int inter,
                                                        int rows, f16* __restrict__ h) {
     const int per_row = inter / 8;
@@ -1510,8 +1497,8 @@ int gemm_f16(qasr_decoder* d, int rows, int n_out, int k, const void* W, const f
         W = d->wdq;
     }
     if (d->own_gemm && qasr::gemm_f16_fits(rows, n_out, k)) {
-        HIP_TRY(qasr::launch_gemm_f16(x, (const f16*)W, y, rows, n_out, k, accumulate, d->ctx->cus,
-                                      d->stream),
+        HIP_TRY(qasr::launch_gemm_f16(x, (const f16*)W, y, rows, n_out, k,
+                                      accumulate ? qasr::kGemmAcc : qasr::kGemmStore, d->ctx->cus, d->stream),
                 "projection GEMM launch");
         return QASR_OK;
     }
@@ -1637,6 +1624,13 @@ int layer_tail(qasr_decoder* d, const qasr_layer_weights& L, int rows, hipStream
         rc = glu_skinny(d, rows, inter, hs, L.gate_up_proj, d->n, d->h, L.gate_up_scale, nullptr,
                         &fused);
         if (rc) return rc;
+    }
+    if (!fused && d->prefill && d->fuse && d->own_gemm && !L.gate_up_scale && qasr::gemm_f16_fits(rows, 2 * inter, hs)) {
+        // A prefill's gate|up: SiLU * up in the GEMM's epilogue.
+        HIP_TRY(qasr::launch_gemm_f16(d->n, (const f16*)L.gate_up_proj, d->h, rows, 2 * inter, hs, qasr::kGemmGlu,
+                                      d->ctx->cus, st),
+                "gate|up GEMM launch");
+        fused = true;
     }
     if (!fused) {
         rc = gemm_f16(d, rows, 2 * inter, hs, L.gate_up_proj, d->n, d->gu, false, L.gate_up_scale);
@@ -2039,7 +2033,7 @@ int qasr_gemm_f16(qasr_ctx* ctx, const void* a_dev, const void* b_dev, void* c_d
     DeviceScope ds(ctx->device);
     if (ds.err != hipSuccess) return hip_fail(ds.err, "hipSetDevice");
     HIP_TRY(qasr::launch_gemm_f16((const f16*)a_dev, (const f16*)b_dev, (f16*)c_dev, m, n, k,
-                                  accumulate != 0, ctx->cus, (hipStream_t)stream),
+                                  accumulate ? qasr::kGemmAcc : qasr::kGemmStore, ctx->cus, (hipStream_t)stream),
             "GEMM launch");
     return QASR_OK;
 }

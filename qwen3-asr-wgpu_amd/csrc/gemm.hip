@@ -1,5 +1,6 @@
 // gemm.hip -- the prefill projections' GEMM on fp16 MFMA (gfx950):
 //   C[m][n] = f16(sum_k A[m][k] * B[n][k]  (+ C[m][n]))
+// or, for gate|up, C[m][n] = f16(SiLU(gate) * up) of the rounded products.
 // A: activation rows [M][K], B: weight rows [N][K] (checkpoint layout), both
 // K-contiguous; f32 accumulation, one rounding of the f32 result (with the
 // residual added in f32 first when accumulating) -- the rounding points of
@@ -76,6 +77,12 @@ __device__ __forceinline__ void dma16_at(const u32x4v& rsrc, int voff, int soff,
                  : "memory");
 }
 
+// kGemmGlu: weight row of B row r of a block whose first column is n0 (of N):
+// groups of 16 gate rows and the up rows of the same 16 columns in turn.
+__device__ __forceinline__ int glu_row(int n0, int r, int N) {
+    return ((r >> 4) & 1) * (N / 2) + n0 / 2 + (r >> 5) * 16 + (r & 15);
+}
+
 // Block coordinates of workgroup bid over nmt row and nnt column blocks (see
 // the XCD note above).
 __device__ __forceinline__ void tile_of(int bid, int nmt, int nnt, int& mt, int& nt) {
@@ -99,9 +106,14 @@ __device__ __forceinline__ void tile_of(int bid, int nmt, int nnt, int& mt, int&
 // and 256 x 256 x 2048 tiles took ~3 us longer each); with the residual the
 // strip is staged in f32 and all its C pieces are requested before the first
 // use (one memory round trip per strip).  Rows past M are not stored.
-template <int MT, int NT, bool ACC>
+// kGemmGlu: the 32 B rows of tile j are 16 gate rows and the same 16 columns'
+// up rows (glu_row), so a lane holds gate in elements 0..7 and up in 8..15 and
+// writes h = f16(SiLU(gate) up), both rounded to f16 first, to columns n0 + 16 j
+// + 8 (e / 4) + 4 g + e % 4, e < 8, of C [M][N / 2].
+template <int MT, int NT, int OUT>
 struct Epilogue {
-    static constexpr int kCols = 32 * NT;
+    static constexpr bool ACC = OUT == kGemmAcc, GLU = OUT == kGemmGlu;
+    static constexpr int kCols = GLU ? 16 * NT : 32 * NT;
     static constexpr int kRow = ACC ? kCols * 4 + 16 : kCols * 2 + 16;  // padded LDS row, bytes
     static constexpr int kBytes = 32 * kRow;                            // per wave
     static constexpr int kPer = kCols / 8;                              // 8-column pieces per row
@@ -123,9 +135,15 @@ struct Epilogue {
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int col = 32 * j + 8 * q + 4 * g;
-                    if constexpr (ACC) {
+                for (int q = 0; q < (GLU ? 2 : 4); ++q) {
+                    const int col = (GLU ? 16 : 32) * j + 8 * q + 4 * g;
+                    if constexpr (GLU) {
+                        half4v h;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            h[e] = f16_of_f32(silu_times((float)(f16)acc[i][j][4 * q + e], (float)(f16)acc[i][j][8 + 4 * q + e]));
+                        *reinterpret_cast<half4v*>(ep + l32 * kRow + col * 2) = h;
+                    } else if constexpr (ACC) {
                         *reinterpret_cast<float4*>(ep + l32 * kRow + col * 4) =
                             make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
                     } else {
@@ -179,7 +197,7 @@ struct Epilogue {
 // every second MFMA, then A.
 constexpr int kBar = 2;
 
-template <int BM, int BN, int NB, bool ACC>
+template <int BM, int BN, int NB, int OUT>
 __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict__ A, const f16* __restrict__ B,
                                                           f16* __restrict__ C, int M, int N, int K) {
     constexpr int MT = BM / 64, NT = BN / 64;
@@ -196,7 +214,7 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict_
     static_assert(kStrA >= 1, "copies fit a step");
     constexpr int kEarlyB = (S - kBar) / 2 < BCOPY ? (S - kBar) / 2 : BCOPY;  // B copies inside slice 3
     __shared__ __attribute__((aligned(16))) char smem[NA * kABuf + NB * kBBuf];
-    static_assert(4 * Epilogue<MT, NT, ACC>::kBytes <= NA * kABuf + NB * kBBuf, "epilogue staging fits");
+    static_assert(4 * Epilogue<MT, NT, OUT>::kBytes <= NA * kABuf + NB * kBBuf, "epilogue staging fits");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int g = lane >> 5, l32 = lane & 31;
@@ -217,7 +235,7 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict_
 #pragma unroll
     for (int j = 0; j < BCOPY; ++j) {
         const int p = 64 * (4 * j + wave) + lane, row = p >> 3;
-        boff[j] = (n0 + row) * K * 2 + slot_of(row, p & 7) * 16;
+        boff[j] = (OUT == kGemmGlu ? glu_row(n0, row, N) : n0 + row) * K * 2 + slot_of(row, p & 7) * 16;
     }
     const uint32_t alds = lds_addr(smem) + wave * 1024, blds = alds + NA * kABuf;
     auto copy_a = [&](int t, int buf, int j) { dma16_at(ares, aoff[j], t * kRowBytes, alds + buf + j * 4096); };
@@ -336,8 +354,8 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict_
     advance();
     step(t, a0, a1, a2, b0, b1, b2, std::integral_constant<int, 8>{});
     __syncthreads();  // every wave is past its last operand reads
-    Epilogue<MT, NT, ACC>::run(acc, smem + wave * Epilogue<MT, NT, ACC>::kBytes, C, M, N, m0 + wm * (BM / 2),
-                               n0 + wn * (BN / 2), lane);
+    Epilogue<MT, NT, OUT>::run(acc, smem + wave * Epilogue<MT, NT, OUT>::kBytes, C, M, OUT == kGemmGlu ? N / 2 : N,
+                               m0 + wm * (BM / 2), (n0 + wn * (BN / 2)) / (OUT == kGemmGlu ? 2 : 1), lane);
 }
 
 // ---- small tiles -------------------------------------------------------------
@@ -348,7 +366,7 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict_
 // read of each 16-k slice under the slice before it waited four LDS latencies:
 // 131 x 1024 x 3072 14.6 -> 11.8 us, 420 x 2048 x 6144 26.2 -> 22.4 us), and
 // NS stages keep NS - 2 steps of copies in flight.
-template <int BM, int BN, int NS, int WGN, bool ACC>
+template <int BM, int BN, int NS, int WGN, int OUT>
 __global__ __launch_bounds__(128 * WGN, 1) void gemm_small_kernel(const f16* __restrict__ A, const f16* __restrict__ B,
                                                                   f16* __restrict__ C, int M, int N, int K) {
     constexpr int kWaves = 2 * WGN;
@@ -363,7 +381,7 @@ __global__ __launch_bounds__(128 * WGN, 1) void gemm_small_kernel(const f16* __r
     static_assert(NS >= 2 && NS <= 6 && (NS - 1) * kStepCopies <= 63, "copy stages");
     constexpr int kABuf = BM * kRowBytes, kBBuf = BN * kRowBytes;
     __shared__ __attribute__((aligned(16))) char smem[NS * (kABuf + kBBuf)];
-    static_assert(kWaves * Epilogue<MT, NT, ACC>::kBytes <= NS * (kABuf + kBBuf), "epilogue staging fits");
+    static_assert(kWaves * Epilogue<MT, NT, OUT>::kBytes <= NS * (kABuf + kBBuf), "epilogue staging fits");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
     const int g = lane >> 5, l32 = lane & 31;
@@ -382,7 +400,7 @@ __global__ __launch_bounds__(128 * WGN, 1) void gemm_small_kernel(const f16* __r
 #pragma unroll
     for (int j = 0; j < BCOPY; ++j) {
         const int p = 64 * (kWaves * j + wave) + lane, row = p >> 3;
-        boff[j] = (n0 + row) * K * 2 + slot_of(row, p & 7) * 16;
+        boff[j] = (OUT == kGemmGlu ? glu_row(n0, row, N) : n0 + row) * K * 2 + slot_of(row, p & 7) * 16;
     }
     const uint32_t alds = lds_addr(smem) + wave * 1024, blds = alds + NS * kABuf;
     auto copy_step = [&](int t, int buf) {
@@ -482,8 +500,8 @@ __global__ __launch_bounds__(128 * WGN, 1) void gemm_small_kernel(const f16* __r
         }
     }
     // Every wave's last operand reads returned before the last step's barrier.
-    Epilogue<MT, NT, ACC>::run(acc, smem + wave * Epilogue<MT, NT, ACC>::kBytes, C, M, N, m0 + wm * WM, n0 + wn * WN,
-                               lane);
+    Epilogue<MT, NT, OUT>::run(acc, smem + wave * Epilogue<MT, NT, OUT>::kBytes, C, M, OUT == kGemmGlu ? N / 2 : N,
+                               m0 + wm * WM, (n0 + wn * WN) / (OUT == kGemmGlu ? 2 : 1), lane);
 }
 
 struct GemmCall {
@@ -491,27 +509,31 @@ struct GemmCall {
     const f16* B;
     f16* C;
     int M, N, K;
-    bool accumulate;
+    GemmOut out;
     hipStream_t stream;
 };
 
 template <int BM, int BN, int NB>
 hipError_t launch_big(const GemmCall& c) {
     const dim3 grid((unsigned)(((c.M + BM - 1) / BM) * (c.N / BN)));
-    if (c.accumulate)
-        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, true>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+    if (c.out == kGemmAcc)
+        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, kGemmAcc>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+    else if (c.out == kGemmGlu)
+        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, kGemmGlu>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     else
-        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, false>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, kGemmStore>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     return hipGetLastError();
 }
 
 template <int BM, int BN, int NS, int WGN>
 hipError_t launch_small(const GemmCall& c) {
     const dim3 grid((unsigned)(((c.M + BM - 1) / BM) * (c.N / BN)));
-    if (c.accumulate)
-        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, true>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+    if (c.out == kGemmAcc)
+        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, kGemmAcc>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+    else if (c.out == kGemmGlu)
+        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, kGemmGlu>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     else
-        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, false>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, kGemmStore>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     return hipGetLastError();
 }
 
@@ -569,11 +591,11 @@ bool gemm_f16_fits(int M, int N, int K) {
            (int64_t)M * K * 2 < (int64_t(1) << 31) && (int64_t)N * K * 2 < (int64_t(1) << 31);
 }
 
-hipError_t launch_gemm_f16(const f16* A, const f16* B, f16* C, int M, int N, int K, bool accumulate,
+hipError_t launch_gemm_f16(const f16* A, const f16* B, f16* C, int M, int N, int K, GemmOut out,
                            int cus, hipStream_t stream) {
     if (!gemm_f16_fits(M, N, K)) return hipErrorInvalidValue;
     const int64_t ncu = std::max(1, cus);
-    GemmCall c{A, B, C, M, N, K, accumulate, stream};
+    GemmCall c{A, B, C, M, N, K, out, stream};
     // QASR_GEMM_TILE = 1..6 forces that tile for all rows (the tests compare
     // them; one whose kernel needs more K steps than there are is not forced).
     const char* forced = std::getenv("QASR_GEMM_TILE");
@@ -609,7 +631,7 @@ hipError_t launch_gemm_f16(const f16* A, const f16* B, f16* C, int M, int N, int
     const hipError_t e = t1->launch(c);
     if (e != hipSuccess || !t2) return e;
     c.A = A + (int64_t)m1 * K;
-    c.C = C + (int64_t)m1 * N;
+    c.C = C + (int64_t)m1 * (out == kGemmGlu ? N / 2 : N);
     c.M = M - m1;
     return t2->launch(c);
 }

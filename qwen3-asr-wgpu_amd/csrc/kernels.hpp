@@ -159,9 +159,12 @@ hipError_t launch_prefill_attn(const PrefillArgs& a, int rows_per_block, const P
 
 // Prefill projections (gemm.hip): C[M][N] = f16(A[M][K] . B[N][K]^T (+ C)),
 // f32 accumulation, row-major, leading dimensions K, K and N, 16-byte
-// aligned.  gemm_f16_fits: K % 64 == 0, N % 256 == 0, both operands < 2 GB.
+// aligned.  kGemmGlu: B holds N / 2 gate rows then N / 2 up rows, and C [M][N / 2]
+// = f16(SiLU(gate) * up) of the two products, each rounded to f16 first.
+// gemm_f16_fits: K % 64 == 0, N % 256 == 0, both operands < 2 GB.
+enum GemmOut : int { kGemmStore, kGemmAcc, kGemmGlu };
 bool gemm_f16_fits(int M, int N, int K);
-hipError_t launch_gemm_f16(const f16* A, const f16* B, f16* C, int M, int N, int K, bool accumulate,
+hipError_t launch_gemm_f16(const f16* A, const f16* B, f16* C, int M, int N, int K, GemmOut out,
                            int cus, hipStream_t stream);
 
 }  // namespace qasr
