@@ -58,26 +58,49 @@ constexpr int kMaxPrefillSegs = 64;  // segments of one batched prefill call
 // workspace (about 61 KB per row at the 1.7B shape, 1 GB at the limit).
 constexpr int kMaxDecoderRows = 16384;
 
-// ---- block reductions (wave64 shuffles, then one LDS pass) ---------------
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m);
-    return v;
+// ---- block reductions (wave64 butterflies, then one LDS pass) ------------
+// v += the value of lane ^ M, without LDS: the halves and the row pairs swap
+// (permlane), inside a 16-lane row DPP moves.  row_ror:4 stands for ^ 4 once
+// the ^ 8 step has made lanes i and i ^ 8 equal.
+template <int M>
+__device__ __forceinline__ float add_xor(float v) {
+    if constexpr (M == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else if constexpr (M == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+        static_assert(M == 8 || M == 4 || M == 2 || M == 1, "butterfly step");
+        return v + qasr::dpp<M == 8 ? qasr::kDppRor8 : M == 4 ? qasr::kDppRor4 : M == 2 ? qasr::kDppXor2 : qasr::kDppXor1>(v);
+    }
 }
 
-// N independent wave_sums, each step's N exchanges issued together (one LDS
-// latency per step instead of one per value).  Each lane adds the same pairs
-// as wave_sum, so every result is bit-identical to wave_sum's.
+// N independent wave sums, each lane adding the pairs of the butterfly 32, 16,
+// .. 1 (every lane gets the total).  A projection's folded norm has up to 16
+// of them in its way to the first MFMA: shuffles through LDS in place of the
+// register moves took the 16-slot 1.7B step 1.0% longer (1809 -> 1789 us with
+// the argmax below moved too), the one-slot 0.6B int8 step 1.8% (974 -> 956).
 template <int N>
 __device__ __forceinline__ void wave_sums(float (&v)[N]) {
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-        float o[N];
+    for (int i = 0; i < N; ++i) v[i] = add_xor<32>(v[i]);
 #pragma unroll
-        for (int i = 0; i < N; ++i) o[i] = __shfl_xor(v[i], m);
+    for (int i = 0; i < N; ++i) v[i] = add_xor<16>(v[i]);
 #pragma unroll
-        for (int i = 0; i < N; ++i) v[i] += o[i];
-    }
+    for (int i = 0; i < N; ++i) v[i] = add_xor<8>(v[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = add_xor<4>(v[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = add_xor<2>(v[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = add_xor<1>(v[i]);
+}
+
+__device__ __forceinline__ float wave_sum(float v) {
+    float u[1] = {v};
+    wave_sums(u);
+    return u[0];
 }
 
 // (value, index) pair order for the argmax: larger value, then smaller index
@@ -86,16 +109,50 @@ __device__ __forceinline__ bool better(float v, int i, float bv, int bi) {
     return v > bv || (v == bv && i < bi);
 }
 
-__device__ __forceinline__ void wave_argmax(float& v, int& i) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-        const float ov = __shfl_xor(v, m);
-        const int oi = __shfl_xor(i, m);
+// One butterfly step of the argmax (moves as in add_xor: every step's operation
+// is symmetric, so the lanes a ror:4 pairs hold equal candidates).
+template <int M>
+__device__ __forceinline__ void argmax_xor(float& v, int& i) {
+    if constexpr (M >= 16) {
+        const uint32_t vb = __float_as_uint(v), ib = (uint32_t)i;
+        float v1;
+        int i1;
+        if constexpr (M == 32) {
+            const auto rv = __builtin_amdgcn_permlane32_swap(vb, vb, false, false);
+            const auto ri = __builtin_amdgcn_permlane32_swap(ib, ib, false, false);
+            v = __uint_as_float(rv[0]), v1 = __uint_as_float(rv[1]), i = (int)ri[0], i1 = (int)ri[1];
+        } else {
+            const auto rv = __builtin_amdgcn_permlane16_swap(vb, vb, false, false);
+            const auto ri = __builtin_amdgcn_permlane16_swap(ib, ib, false, false);
+            v = __uint_as_float(rv[0]), v1 = __uint_as_float(rv[1]), i = (int)ri[0], i1 = (int)ri[1];
+        }
+        if (better(v1, i1, v, i)) {
+            v = v1;
+            i = i1;
+        }
+    } else {
+        constexpr int kCtrl = M == 8 ? qasr::kDppRor8 : M == 4 ? qasr::kDppRor4 : M == 2 ? qasr::kDppXor2 : qasr::kDppXor1;
+        const float ov = qasr::dpp<kCtrl>(v);
+        const int oi = __builtin_amdgcn_update_dpp(0, i, kCtrl, 0xf, 0xf, false);
         if (better(ov, oi, v, i)) {
             v = ov;
             i = oi;
         }
     }
+}
+
+// The best candidate of each 16-lane row, in every lane of the row.
+__device__ __forceinline__ void row_argmax(float& v, int& i) {
+    argmax_xor<8>(v, i);
+    argmax_xor<4>(v, i);
+    argmax_xor<2>(v, i);
+    argmax_xor<1>(v, i);
+}
+
+__device__ __forceinline__ void wave_argmax(float& v, int& i) {
+    argmax_xor<32>(v, i);
+    argmax_xor<16>(v, i);
+    row_argmax(v, i);
 }
 
 // ---- kernels -------------------------------------------------------------
@@ -475,7 +532,21 @@ struct NormPrologue {
             *(float4*)&s_gain[8 * c + 4] =
                 make_float4((float)gain.e[4], (float)gain.e[5], (float)gain.e[6], (float)gain.e[7]);
         }
-        wave_sums(v);
+        // The butterflies of existing rows only (wave-uniform; one row's four
+        // sums are one per wave): sixteen for one row took the one-slot 0.6B
+        // int8 step 2.3% longer (986 against 964 us).
+        if (4 * p.M <= KS) {
+            float u[1] = {v[0]};
+            wave_sums(u);
+            v[0] = u[0];
+        } else if (4 * p.M <= 4 * KS && kPer > 4) {
+            float u[4] = {v[0], v[1], v[2], v[3]};
+            wave_sums(u);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = u[i];
+        } else {
+            wave_sums(v);
+        }
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             const int q = wave + i * KS;
@@ -532,7 +603,7 @@ __device__ __forceinline__ void skinny_tile_out(const SkinnyArgs& p, qasr::float
             // Lanes r and r^8 (same rows) exchange gate and up; every lane of
             // the wave takes part in the shuffle.
             const float v = (float)(f16)sum[i];
-            const float up = __shfl_xor(v, 8);
+            const float up = qasr::dpp<qasr::kDppRor8>(v);  // lane ^ 8 of the row
             if (r < 8 && m < M)
                 ((f16*)p.Y)[(int64_t)m * (N / 2) + 8 * tile + r] = f16_of_f32(silu_times(v, up));
             continue;
@@ -562,15 +633,7 @@ __device__ __forceinline__ void skinny_tile_out(const SkinnyArgs& p, qasr::float
                     bv = sum[i];
                     bi = n;
                 }
-#pragma unroll
-                for (int msk = 8; msk >= 1; msk >>= 1) {
-                    const float ov = __shfl_xor(bv, msk);
-                    const int oi = __shfl_xor(bi, msk);
-                    if (better(ov, oi, bv, bi)) {
-                        bv = ov;
-                        bi = oi;
-                    }
-                }
+                row_argmax(bv, bi);
                 const int m = 4 * g + i;
                 if (r == 0 && m < M) {
                     p.am_v[(int64_t)m * (N / 16) + tile] = bv;

@@ -468,6 +468,14 @@ def test_fused_epilogues_equal_unfused(gpu, model, batch, int8, lds, monkeypatch
     assert np.array_equal(out["fused"][1], out["unfused"][1])
 
 
+@pytest.mark.parametrize("model,batch", [("0.6B", 6), ("0.6B", 8), ("1.7B", 9), ("0.6B", 12), ("1.7B", 13)])
+def test_folded_norm_row_counts(gpu, model, batch, monkeypatch):
+    """The folded norm reduces only the rows there are, by one, four or all of
+    a wave's sums: row counts on both sides of each choice (waves of 4, 8 and
+    12 to a workgroup), bitwise as the norm kernel."""
+    test_fused_epilogues_equal_unfused(gpu, model, batch, False, "1", monkeypatch)
+
+
 @pytest.mark.parametrize("model,batch", [("1.7B", 16), ("0.6B", 1), ("0.6B", 9), ("1.7B", 3)])
 def test_argmax_from_logits_tiles_equals_two_pass(gpu, model, batch, monkeypatch):
     """The greedy token from the logits kernel's per-tile candidates
