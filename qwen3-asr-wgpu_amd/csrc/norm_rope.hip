@@ -124,6 +124,88 @@ __global__ __launch_bounds__(kRowThreads) void norm_rope_append_kernel(
     }
 }
 
+// The same rows for many of them, one wave per row and no workgroup: what
+// counts then is how many rows a CU holds and how little each does, not one
+// row's latency.  Every load of the row is in flight at once; a lane holds a
+// piece of 8 dims and its rotation partner in registers, so each normed value
+// is made once for both outputs; only the heads' serial sums pass through
+// LDS, as f16 (6.4 KB a row against 20 KB).  Against the kernel above, us:
+// 1,024 rows 7.7 -> 6.8, 16 segments of 80 rows 10.8 -> 8.1, 16 of 267 rows
+// 24.5 -> 20.2 (70 MB); 420 rows 4.9 -> 5.1, one 3.65 -> 4.05 (the single wave
+// does a row's work in series).
+// NP: piece pairs per lane, ceil((nqh + nkvh) * 8 / 64).
+constexpr int kManyRows = 800;
+template <int NP>
+__global__ __launch_bounds__(64) void norm_rope_many_kernel(
+    CacheGeom g, int layer, SegPlan P, const f16* __restrict__ qkv,
+    const f16* __restrict__ q_gain, const f16* __restrict__ k_gain,
+    const f16* __restrict__ cos_tab, const f16* __restrict__ sin_tab, f16* __restrict__ q_out) {
+    constexpr int kHeads = 8 * NP;
+    constexpr int NV = (kHeads / 3 * 16 + 63) / 64;  // V pieces per lane (nqh = 2 nkvh)
+    __shared__ __attribute__((aligned(16))) f16 s_raw[kHeads * kPad];
+
+    const int row = blockIdx.x, lane = threadIdx.x;
+    const int nqh = P.nqh, nkvh = g.nkvh, nh = nqh + nkvh;
+    const f16* src = qkv + (int64_t)row * ((int64_t)(nqh + 2 * nkvh) * kHeadDim);
+    // Lane l, pair k: head l / 8 + 8 k, pieces w = l % 8 and w + 8.  Heads past
+    // the last read the last one (their outputs are not stored).
+    const int w = lane & 7, h0 = lane >> 3;
+    H8 x[NP][2], v[NV];
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        const f16* hs = src + min(h0 + 8 * k, nh - 1) * kHeadDim + 8 * w;
+        x[k][0].u = *(const uint4*)hs;
+        x[k][1].u = *(const uint4*)(hs + kHeadDim / 2);
+    }
+    const int nv = nkvh * 16;  // 16-byte V pieces
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k].u = *(const uint4*)(src + (int64_t)nh * kHeadDim + min(lane + 64 * k, nv - 1) * 8);
+    // The row's segment: the number of later segment starts at or before it
+    // (lane i reads segment i's fields; the arrays hold 64).
+    static_assert(kMaxBatch == 64, "one lane per segment");
+    const int e_slot = P.slot[lane], e_pos = P.pos0[lane], e_r0 = P.row_base[lane], e_r1 = P.row_base[lane + 1];
+    const int sg = __popcll(__ballot(lane + 1 < P.nseg && e_r1 <= row));
+    const int pos = __builtin_amdgcn_readlane(e_pos, sg) + row - __builtin_amdgcn_readlane(e_r0, sg);
+    f16* kdst = g.base + __builtin_amdgcn_readlane(e_slot, sg) * g.slot_stride + layer * g.layer_stride +
+                (int64_t)pos * kHeadDim;
+    f16* vdst = kdst + g.kv_stride;
+    H8 c[2], sn[2], gn[NP][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int d = 8 * w + i * (kHeadDim / 2);
+        c[i].u = *(const uint4*)(cos_tab + (int64_t)pos * kHeadDim + d);
+        sn[i].u = *(const uint4*)(sin_tab + (int64_t)pos * kHeadDim + d);
+#pragma unroll
+        for (int k = 0; k < NP; ++k) gn[k][i].u = *(const uint4*)((h0 + 8 * k < nqh ? q_gain : k_gain) + d);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // every load is requested before the first use
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        f16* d = &s_raw[(h0 + 8 * k) * kPad + 8 * w];
+        *(uint4*)d = x[k][0].u;
+        *(uint4*)(d + kHeadDim / 2) = x[k][1].u;
+    }
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        const int it = lane + 64 * k;
+        if (it < nv) *(uint4*)(vdst + (it >> 4) * g.head_stride + (it & 15) * 8) = v[k].u;
+    }
+    __syncthreads();  // one wave: its LDS writes have completed
+    float inv = 0.0f;
+    if (lane < kHeads) inv = head_inv_rms(&s_raw[lane * kPad], P.eps);
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        const int h = h0 + 8 * k;
+        H8 o[2];
+        rope16(x[k], gn[k], c, sn, __shfl(inv, h), o);
+        if (h < nh) {
+            f16* dst = h < nqh ? q_out + ((int64_t)row * nqh + h) * kHeadDim : kdst + (h - nqh) * g.head_stride;
+            *(uint4*)(dst + 8 * w) = o[0].u;
+            *(uint4*)(dst + 8 * w + kHeadDim / 2) = o[1].u;
+        }
+    }
+}
+
 }  // namespace
 
 hipError_t launch_norm_rope_append(const CacheGeom& g, int layer, const SegPlan& P,
@@ -136,6 +218,17 @@ hipError_t launch_norm_rope_append(const CacheGeom& g, int layer, const SegPlan&
         return hipErrorInvalidValue;
     const int nqk = (P.nqh + g.nkvh) * 16;
     static_assert(kMaxNormHeads * 16 <= 2 * kRowThreads, "two q/k pieces per thread at most");
+    // Many rows: one wave per row (768 rows of one segment take 6.1 us either
+    // way, 900 take 7.4 against 6.6, 16 segments of 50 rows 8.3 against 6.4).
+    if (rows >= kManyRows && P.nqh == kRep * g.nkvh) {
+        if (P.nqh + g.nkvh <= 24)
+            hipLaunchKernelGGL(norm_rope_many_kernel<3>, dim3(rows), dim3(64), 0, stream, g, layer, P, qkv, q_gain,
+                               k_gain, cos_tab, sin_tab, q_out);
+        else
+            hipLaunchKernelGGL(norm_rope_many_kernel<6>, dim3(rows), dim3(64), 0, stream, g, layer, P, qkv, q_gain,
+                               k_gain, cos_tab, sin_tab, q_out);
+        return hipGetLastError();
+    }
     if (nqk <= kRowThreads)
         hipLaunchKernelGGL(norm_rope_append_kernel<1>, dim3(rows), dim3(kRowThreads), 0, stream, g,
                            layer, P, qkv, q_gain, k_gain, cos_tab, sin_tab, q_out);

@@ -35,6 +35,27 @@ __device__ __forceinline__ float head_inv_rms_squares_all(const float* sq, float
     return 1.0f / sqrtf(sum2 / (float)kHeadDim + eps);
 }
 
+// The same sum straight from the head's f16 values in LDS: the square of an
+// f16 is exact in f32, so v_fma_mix_f32 (f16 factors, f32 sum, one rounding)
+// rounds exactly where the reference's product-then-add does.
+__device__ __forceinline__ float head_inv_rms(const f16* raw, float eps) {
+#pragma clang fp contract(off)
+    H8 v[kHeadDim / 8];
+#pragma unroll
+    for (int i = 0; i < kHeadDim / 8; ++i) v[i].u = *(const uint4*)(raw + 8 * i);
+    float sum2 = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kHeadDim / 8; ++i) {
+        const uint32_t d[4] = {v[i].u.x, v[i].u.y, v[i].u.z, v[i].u.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            asm("v_fma_mix_f32 %0, %1, %1, %0 op_sel_hi:[1,1,0]" : "+v"(sum2) : "v"(d[e]));
+            asm("v_fma_mix_f32 %0, %1, %1, %0 op_sel:[1,1,0] op_sel_hi:[1,1,0]" : "+v"(sum2) : "v"(d[e]));
+        }
+    }
+    return 1.0f / sqrtf(sum2 / (float)kHeadDim + eps);
+}
+
 // One roped element j of a head whose raw values, gains and cos/sin rows are
 // given (all f16).  `inv` is the head's inverse RMS.
 __device__ __forceinline__ f16 rope_elem(const f16* raw, const f16* gain, const f16* cos_row,
@@ -75,6 +96,21 @@ __device__ __forceinline__ uint4 rope8(const f16* raw, const f16* gain, const f1
         o.e[e] = f2h(lo ? a - b : a + b);
     }
     return o.u;
+}
+
+// Elements j0 .. j0+7 and their rotation partners j0+64 .. (index 1 of each
+// operand), all operands in registers: per element the arithmetic of
+// rope_elem, each normed value made once for both outputs.
+__device__ __forceinline__ void rope16(const H8 (&x)[2], const H8 (&g)[2], const H8 (&c)[2], const H8 (&sn)[2],
+                                       float inv, H8 (&o)[2]) {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float lo = (h2f(x[0].e[e]) * inv) * h2f(g[0].e[e]);
+        const float hi = (h2f(x[1].e[e]) * inv) * h2f(g[1].e[e]);
+        o[0].e[e] = f2h(lo * h2f(c[0].e[e]) - hi * h2f(sn[0].e[e]));
+        o[1].e[e] = f2h(hi * h2f(c[1].e[e]) + lo * h2f(sn[1].e[e]));
+    }
 }
 
 }  // namespace qasr

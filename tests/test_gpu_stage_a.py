@@ -102,3 +102,52 @@ def test_stage_a_extreme_inputs_bitexact(O, gpu):
     k_ref, _ = ref.cache_f16()
     assert np.array_equal(k_gpu, k_ref)
     g.close()
+
+
+@pytest.mark.parametrize("nqh,nkvh", [(16, 8), (2, 1), (10, 5), (32, 16)])
+@pytest.mark.parametrize("segments", [[(0, 0, 800)], [(1, 37, 801), (0, 5, 3)],
+                                      [(i, 11 * i, 1 + 13 * i) for i in range(12)]])
+def test_many_rows_equal_few_rows(gpu, nqh, nkvh, segments):
+    """From 800 rows one wave does a row; below, a workgroup does.  Both round
+    where the reference rounds, so one call of many rows gives, bit for bit,
+    what calls of a few rows each give, subnormal, large and all-zero heads
+    among them."""
+    import torch
+
+    import qasr_attn
+    from gpu_helpers import say
+
+    hd = 128
+    rows = sum(n for _, _, n in segments)
+    slots = max(s for s, _, _ in segments) + 1
+    g = torch.Generator(device="cuda").manual_seed(81 + nqh + rows)
+    qkv = torch.randn((rows, (nqh + 2 * nkvh) * hd), generator=g, device="cuda").half()
+    qkv[1::7, :hd] *= 2.0 ** -20   # subnormal f16
+    qkv[2::7, hd:2 * hd] *= 1000.0
+    qkv[3::7, :hd] = 0
+    gains = [(torch.randn(hd, generator=g, device="cuda") * 0.1 + 1).half() for _ in range(2)]
+    cos, sin = qasr_attn.mrope_text_tables(2048)
+    ctx = qasr_attn.Context(nqh, nkvh, hd, 1, 1e-6, 2048, 0)
+    ctx.set_rope_tables(cos, sin)
+    got = []
+    for chunk in (10 ** 9, 150):
+        kv = qasr_attn.KVPool(ctx, slots, 1024)
+        kv.tensor().zero_()
+        q = torch.empty((rows, nqh * hd), dtype=torch.float16, device="cuda")
+        say(f"stage (a) {nqh}+{nkvh} heads, {rows} rows, {len(segments)} segments, calls of {chunk}")
+        if chunk > rows:
+            qasr_attn.qk_norm_rope_append(ctx, kv, 0, segments, qkv, *gains, q)
+        else:
+            r0 = 0
+            for slot, pos, n in segments:
+                for a in range(0, n, chunk):
+                    m = min(chunk, n - a)
+                    qasr_attn.qk_norm_rope_append(ctx, kv, 0, [(slot, pos + a, m)], qkv[r0 + a:r0 + a + m],
+                                                  *gains, q[r0 + a:r0 + a + m])
+                r0 += n
+        torch.cuda.synchronize()
+        got.append((q.view(torch.int16).cpu(), kv.tensor().clone().view(torch.int16).cpu()))
+        kv.close()
+    ctx.close()
+    assert torch.equal(got[0][0], got[1][0])
+    assert torch.equal(got[0][1], got[1][1])
