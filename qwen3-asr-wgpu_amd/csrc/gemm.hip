@@ -548,16 +548,26 @@ struct Tile {
     int bm, bn, occ;
     float fix, step[2];
     int min_steps;  // K steps the kernel needs
-    hipError_t (*launch)(const GemmCall&);
 };
-const Tile kTiles[] = {{256, 256, 1, 6.5f, {1.50f, 0.0f}, 2, launch_big<256, 256, 2>},
-                       {192, 256, 1, 6.0f, {1.10f, 0.0f}, 2, launch_big<192, 256, 2>},
-                       {128, 256, 1, 5.5f, {0.82f, 0.0f}, 3, launch_big<128, 256, 3>},
-                       {64, 128, 2, 4.0f, {0.40f, 0.62f}, 1, launch_small<64, 128, 3, 2>},
-                       {128, 64, 2, 4.0f, {0.38f, 0.62f}, 1, launch_small<128, 64, 3, 2>},
-                       {64, 64, 2, 3.5f, {0.25f, 0.44f}, 1, launch_small<64, 64, 4, 2>}};
+const Tile kTiles[] = {{256, 256, 1, 6.5f, {1.50f, 0.0f}, 2},
+                       {192, 256, 1, 6.0f, {1.10f, 0.0f}, 2},
+                       {128, 256, 1, 5.5f, {0.82f, 0.0f}, 3},
+                       {64, 128, 2, 4.0f, {0.40f, 0.62f}, 1},
+                       {128, 64, 2, 4.0f, {0.38f, 0.62f}, 1},
+                       {64, 64, 2, 3.5f, {0.25f, 0.44f}, 1}};
 constexpr int kNumTiles = (int)(sizeof kTiles / sizeof kTiles[0]);
 constexpr float kSecondLaunchUs = 2.0f;
+
+hipError_t launch_tile(const Tile& t, const GemmCall& c) {
+    switch (&t - kTiles) {
+        case 0: return launch_big<256, 256, 2>(c);
+        case 1: return launch_big<192, 256, 2>(c);
+        case 2: return launch_big<128, 256, 3>(c);
+        case 3: return launch_small<64, 128, 3, 2>(c);
+        case 4: return launch_small<128, 64, 3, 2>(c);
+        default: return launch_small<64, 64, 4, 2>(c);
+    }
+}
 
 float tile_us(const Tile& c, int64_t rows, int N, int K, int64_t cus) {
     const int64_t tiles = (rows + c.bm - 1) / c.bm * (N / c.bn);
@@ -600,7 +610,7 @@ hipError_t launch_gemm_f16(const f16* A, const f16* B, f16* C, int M, int N, int
     // them; one whose kernel needs more K steps than there are is not forced).
     const char* forced = std::getenv("QASR_GEMM_TILE");
     const int f = forced ? std::atoi(forced) : 0;
-    if (f >= 1 && f <= kNumTiles && K / kBK >= kTiles[f - 1].min_steps) return kTiles[f - 1].launch(c);
+    if (f >= 1 && f <= kNumTiles && K / kBK >= kTiles[f - 1].min_steps) return launch_tile(kTiles[f - 1], c);
     // One tile for all rows, or a tile's whole rounds for the first rows and a
     // second launch with the best tile for the rest, whichever the model calls
     // fastest: 4,269 rows of gate|up are 816 tiles of 256 x 256, 3.2 rounds
@@ -628,12 +638,12 @@ hipError_t launch_gemm_f16(const f16* A, const f16* B, f16* C, int M, int N, int
         }
     }
     c.M = m1;
-    const hipError_t e = t1->launch(c);
+    const hipError_t e = launch_tile(*t1, c);
     if (e != hipSuccess || !t2) return e;
     c.A = A + (int64_t)m1 * K;
     c.C = C + (int64_t)m1 * (out == kGemmGlu ? N / 2 : N);
     c.M = M - m1;
-    return t2->launch(c);
+    return launch_tile(*t2, c);
 }
 
 }  // namespace qasr
