@@ -22,8 +22,8 @@
 // does not depend on the row count, so a prompt prefilled alone and inside a
 // batch gives the same bits (the library's stream-K kernels split K by the
 // row count).  QASR_PREFILL_GEMM=blas sends them to rocBLAS instead (beta = 1
-// for the residual; measured 1.4-2.5x faster at these shapes, not row
-// invariant).  The elementwise steps are small HIP kernels below.  Nothing here allocates per
+// for the residual; not row invariant).  A prefill's SiLU * up is the gate|up
+// GEMM's epilogue, and its int8 projections are dequantised once per layer.  The elementwise steps are small HIP kernels below.  Nothing here allocates per
 // call: the activation workspace is sized for max_rows at creation, and
 // rocBLAS gets a fixed workspace so that a step can be captured in a graph.
 

@@ -1,5 +1,5 @@
 // norm_rope.hip -- stage (a): fused q/k RMSNorm + rotate-half MRoPE + f16 KV
-// append, one workgroup per row.
+// append, one workgroup per row (one wave from kManyRows rows).
 //
 // Replaces the reference's qkv_extract / qkv_extract_slots WGSL kernels
 // (src/shaders.rs:1376-1635) with the numerics of the CPU decoder

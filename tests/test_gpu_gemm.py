@@ -95,7 +95,7 @@ def g_ctx():
 
 
 # Block tiles the launcher chooses from (QASR_GEMM_TILE = 1..6): 256x256,
-# 192x256 and 128x128 (eight waves), 64x128, 128x64, 64x64 (four).
+# 192x256, 128x256, 64x128, 128x64, 64x64 (four waves each).
 TILES = [1, 2, 3, 4, 5, 6]
 
 
@@ -107,8 +107,8 @@ def test_gemm_tile_choice_keeps_bits(gpu, m, n, k, accumulate, monkeypatch):
     (a function of the row count) cannot make a row's result depend on how
     many rows the call carries; the default choice is one of them, and the
     shared result meets the fp32 reference's bound.  K = 64 and 128 run the
-    large tiles' ping-pong loop over one and two K steps (its copies and
-    waits at their boundaries)."""
+    tiles' loops over one and two K steps (their copies and waits at the
+    boundaries)."""
     import torch
 
     import qasr_attn
