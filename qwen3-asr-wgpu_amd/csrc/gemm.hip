@@ -9,7 +9,7 @@
 //
 // Two kernels of one design, for tiles of 128 x 256 and more (gemm_big_kernel)
 // and down to 64 x 64 (gemm_small_kernel); launch_gemm_f16 chooses per shape by
-// a cost model.  K steps of 64; waves in a 2 x n grid, each computing tiles of
+// a cost model.  K steps of 64; four waves, each computing tiles of
 // v_mfma_f32_32x32x16_f16 as D = B A^T, so that a lane ends with four
 // consecutive columns of a row.  Both operand tiles go global -> LDS by direct
 // copies (buffer_load ... lds, one 1 KB block per wave instruction) into a ring
@@ -28,7 +28,7 @@
 // from HBM, against the two-stage ping-pong and slice-by-slice loops these
 // kernels replace): 4269 x 12288 x 2048 207 -> 189, 4269 x 4096 x 2048 83 -> 68,
 // 4269 x 2048 x 2048 + residual 48 -> 41, 4269 x 2048 x 6144 + residual 138 ->
-// 112, 420 x 12288 x 2048 36.7 -> 31.5, 420 x 4096 x 2048 18.7 -> 15.8,
+// 107, 420 x 12288 x 2048 36.7 -> 31.5, 420 x 4096 x 2048 18.7 -> 15.8,
 // 420 x 2048 x 2048 + residual 10.9 -> 9.6, 131 x 1024 x 3072 + residual 14.5 ->
 // 11.7; weights in the memory-side cache, 420 x 2048 x 6144 + residual 25.7 -> 21.9.
 
@@ -178,8 +178,10 @@ struct Epilogue {
 };
 
 // ---- large tiles -------------------------------------------------------------
-// Four waves in a 2 x 2 grid, one per SIMD, each (BM/2) x (BN/2): the largest
-// wave tile, so the fewest LDS operand bytes per MFMA.  What bounds it is the
+// Four waves in a WGM x (4 / WGM) grid, one per SIMD: 2 x 2, the largest wave
+// tile, so the fewest LDS operand bytes per MFMA, or 1 x 4 for 160 rows (five
+// 32-row tiles a wave; 4,269 rows of 2,048 columns are then 216 blocks of 256
+// CUs, not 184 of 192 rows: K = 6144 with the residual 112-115 -> 107 us).  What bounds it is the
 // copies: a CU takes in at most ~85 GB/s of them (a copy-only loop of these
 // tiles), 0.75 us for the 64 KB of a 256 x 256 step against 0.85 us of MFMAs,
 // so they have to run all the time.  With two stages of both operands they
@@ -197,10 +199,12 @@ struct Epilogue {
 // every second MFMA, then A.
 constexpr int kBar = 2;
 
-template <int BM, int BN, int NB, int OUT>
+template <int BM, int BN, int NB, int WGM, int OUT>
 __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict__ A, const f16* __restrict__ B,
                                                           f16* __restrict__ C, int M, int N, int K) {
-    constexpr int MT = BM / 64, NT = BN / 64;
+    constexpr int WGN = 4 / WGM, WM = BM / WGM, WN = BN / WGN;
+    constexpr int MT = WM / 32, NT = WN / 32;
+    static_assert(MT * 32 * WGM == BM && NT * 32 * WGN == BN, "wave tile of whole 32 x 32 MFMA tiles");
     constexpr int ACOPY = BM / 32, BCOPY = BN / 32;  // copies per wave and step
     constexpr int S = MT * NT;                       // MFMAs per slice
     constexpr int NA = 3;
@@ -216,7 +220,7 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict_
     __shared__ __attribute__((aligned(16))) char smem[NA * kABuf + NB * kBBuf];
     static_assert(4 * Epilogue<MT, NT, OUT>::kBytes <= NA * kABuf + NB * kBBuf, "epilogue staging fits");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / WGN, wn = wave % WGN;
     const int g = lane >> 5, l32 = lane & 31;
     int mt, nt;
     tile_of(blockIdx.x, (M + BM - 1) / BM, N / BN, mt, nt);
@@ -245,7 +249,7 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict_
     int ao[kSlices], bo[kSlices];
 #pragma unroll
     for (int ks = 0; ks < kSlices; ++ks) {
-        const int ra = wm * (BM / 2) + l32, rb = wn * (BN / 2) + l32;
+        const int ra = wm * WM + l32, rb = wn * WN + l32;
         ao[ks] = ra * kRowBytes + slot_of(ra, 2 * ks + g) * 16;
         bo[ks] = NA * kABuf + rb * kRowBytes + slot_of(rb, 2 * ks + g) * 16;
     }
@@ -355,7 +359,7 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict_
     step(t, a0, a1, a2, b0, b1, b2, std::integral_constant<int, 8>{});
     __syncthreads();  // every wave is past its last operand reads
     Epilogue<MT, NT, OUT>::run(acc, smem + wave * Epilogue<MT, NT, OUT>::kBytes, C, M, OUT == kGemmGlu ? N / 2 : N,
-                               m0 + wm * (BM / 2), (n0 + wn * (BN / 2)) / (OUT == kGemmGlu ? 2 : 1), lane);
+                               m0 + wm * WM, (n0 + wn * WN) / (OUT == kGemmGlu ? 2 : 1), lane);
 }
 
 // ---- small tiles -------------------------------------------------------------
@@ -513,15 +517,15 @@ struct GemmCall {
     hipStream_t stream;
 };
 
-template <int BM, int BN, int NB>
+template <int BM, int BN, int NB, int WGM>
 hipError_t launch_big(const GemmCall& c) {
     const dim3 grid((unsigned)(((c.M + BM - 1) / BM) * (c.N / BN)));
     if (c.out == kGemmAcc)
-        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, kGemmAcc>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, WGM, kGemmAcc>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     else if (c.out == kGemmGlu)
-        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, kGemmGlu>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, WGM, kGemmGlu>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     else
-        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, kGemmStore>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+        hipLaunchKernelGGL((gemm_big_kernel<BM, BN, NB, WGM, kGemmStore>), grid, dim3(256), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     return hipGetLastError();
 }
 
@@ -542,6 +546,7 @@ hipError_t launch_small(const GemmCall& c) {
 // of one per CU; the small ones take step[0] alone and step[1] two to a CU
 // (in between, as the square root of the share of CUs with two), and fill in
 // behind each other, so a last part round costs little more than its share.
+// 160 x 256 was fitted at its K = 2048 and 6144 times with most CUs busy.
 // The figures are sweeps of every tile over the 1.7B and 0.6B projections at 64
 // to 4,269 rows and a 16384 x 12288 x 2048 product, weights coming from HBM.
 struct Tile {
@@ -554,18 +559,20 @@ const Tile kTiles[] = {{256, 256, 1, 6.5f, {1.50f, 0.0f}, 2},
                        {128, 256, 1, 5.5f, {0.82f, 0.0f}, 3},
                        {64, 128, 2, 4.0f, {0.40f, 0.62f}, 1},
                        {128, 64, 2, 4.0f, {0.38f, 0.62f}, 1},
-                       {64, 64, 2, 3.5f, {0.25f, 0.44f}, 1}};
+                       {64, 64, 2, 3.5f, {0.25f, 0.44f}, 1},
+                       {160, 256, 1, 10.0f, {1.02f, 0.0f}, 3}};
 constexpr int kNumTiles = (int)(sizeof kTiles / sizeof kTiles[0]);
 constexpr float kSecondLaunchUs = 2.0f;
 
 hipError_t launch_tile(const Tile& t, const GemmCall& c) {
     switch (&t - kTiles) {
-        case 0: return launch_big<256, 256, 2>(c);
-        case 1: return launch_big<192, 256, 2>(c);
-        case 2: return launch_big<128, 256, 3>(c);
+        case 0: return launch_big<256, 256, 2, 2>(c);
+        case 1: return launch_big<192, 256, 2, 2>(c);
+        case 2: return launch_big<128, 256, 3, 2>(c);
         case 3: return launch_small<64, 128, 3, 2>(c);
         case 4: return launch_small<128, 64, 3, 2>(c);
-        default: return launch_small<64, 64, 4, 2>(c);
+        case 5: return launch_small<64, 64, 4, 2>(c);
+        default: return launch_big<160, 256, 3, 1>(c);
     }
 }
 
@@ -606,7 +613,7 @@ hipError_t launch_gemm_f16(const f16* A, const f16* B, f16* C, int M, int N, int
     if (!gemm_f16_fits(M, N, K)) return hipErrorInvalidValue;
     const int64_t ncu = std::max(1, cus);
     GemmCall c{A, B, C, M, N, K, out, stream};
-    // QASR_GEMM_TILE = 1..6 forces that tile for all rows (the tests compare
+    // QASR_GEMM_TILE = 1..7 forces that tile for all rows (the tests compare
     // them; one whose kernel needs more K steps than there are is not forced).
     const char* forced = std::getenv("QASR_GEMM_TILE");
     const int f = forced ? std::atoi(forced) : 0;

@@ -94,9 +94,9 @@ def g_ctx():
     return _CTX
 
 
-# Block tiles the launcher chooses from (QASR_GEMM_TILE = 1..6): 256x256,
-# 192x256, 128x256, 64x128, 128x64, 64x64 (four waves each).
-TILES = [1, 2, 3, 4, 5, 6]
+# Block tiles the launcher chooses from (QASR_GEMM_TILE = 1..7): 256x256,
+# 192x256, 128x256, 64x128, 128x64, 64x64, 160x256 (four waves each).
+TILES = [1, 2, 3, 4, 5, 6, 7]
 
 
 @pytest.mark.parametrize("m,n,k,accumulate", [(300, 512, 256, False), (4269, 2048, 2048, True),
@@ -144,7 +144,7 @@ def test_gemm_tile_choice_keeps_bits(gpu, m, n, k, accumulate, monkeypatch):
 # large tiles' copy stages (2 .. 7, odd ones among them), one row more and less
 # than a block, and a row count that takes a second launch for its last rows.
 EDGES = [(255, 256, 192), (257, 256, 256), (129, 512, 320), (385, 768, 448), (1, 256, 384),
-         (4096 + 37, 4096, 256), (513, 12288, 128)]
+         (4096 + 37, 4096, 256), (513, 12288, 128), (161, 512, 256)]
 
 
 @pytest.mark.parametrize("m,n,k", EDGES)
