@@ -370,7 +370,16 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict_
 // read of each 16-k slice under the slice before it waited four LDS latencies:
 // 131 x 1024 x 3072 14.6 -> 11.8 us, 420 x 2048 x 6144 26.2 -> 22.4 us), and
 // NS stages keep NS - 2 steps of copies in flight.
-template <int BM, int BN, int NS, int WGN, int OUT>
+// SLICED: each slice is read under the MFMAs of the slice before it.  Where
+// some CUs have two workgroups, the other one covers the LDS latencies and
+// whole-step reads only queue up behind each other.  64 x 64 tiles, one to 1.5
+// a CU, whole-step reads -> slices, us, weights from HBM and (in brackets) in the
+// memory-side cache: 576 x 2048 x 2048 + residual 14.7 -> 13.9 (13.1 -> 11.7),
+// 576 x 2048 x 6144 + residual 39.5 -> 37.7 (36.8 -> 36.3), 192 x 6144 x 1024 11.1 ->
+// 10.9 (7.7 -> 7.3); only with few row blocks and weights from HBM are slices slower:
+// 384 x 4096 x 2048 17.4 -> 17.9 (13.3 -> 12.2).  At one tile a CU (495 x 2048 x 2048
+// 11.3 (9.4) -> 11.4 (10.6)) and near two (1007 rows 18.2 -> 18.5) whole steps are faster.
+template <int BM, int BN, int NS, int WGN, bool SLICED, int OUT>
 __global__ __launch_bounds__(128 * WGN, 1) void gemm_small_kernel(const f16* __restrict__ A, const f16* __restrict__ B,
                                                                   f16* __restrict__ C, int M, int N, int K) {
     constexpr int kWaves = 2 * WGN;
@@ -421,39 +430,11 @@ __global__ __launch_bounds__(128 * WGN, 1) void gemm_small_kernel(const f16* __r
         ao[ks] = ra * kRowBytes + slot_of(ra, 2 * ks + g) * 16;
         bo[ks] = NS * kABuf + rb * kRowBytes + slot_of(rb, 2 * ks + g) * 16;
     }
-    half8v fa[2][kSlices][MT], fb[2][kSlices][NT];
-    // The addresses step to the next stage (buf + 1, or back to 0) in place: an
-    // address made in a register the MFMAs in flight still read would wait for
-    // them (420 x 2048 x 6144: 25 against 21.5 us).
-    auto read_step = [&](int buf, int q) {
-        const int da = buf == NS - 1 ? -(NS - 1) * kABuf : kABuf;
-        const int db = buf == NS - 1 ? -(NS - 1) * kBBuf : kBBuf;
-#pragma unroll
-        for (int ks = 0; ks < kSlices; ++ks) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i) fa[q][ks][i] = *(const half8v*)(smem + ao[ks] + i * 4096);
-#pragma unroll
-            for (int i = 0; i < NT; ++i) fb[q][ks][i] = *(const half8v*)(smem + bo[ks] + i * 4096);
-            ao[ks] += da;
-            bo[ks] += db;
-            asm volatile("" : "+v"(ao[ks]), "+v"(bo[ks]));
-        }
-    };
     float16v acc[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = (float16v){};
-    auto mfma_step = [&](int q) {
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int ks = 0; ks < kSlices; ++ks)
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = mfma32(fb[q][ks][j], fa[q][ks][i], acc[i][j]);  // D = B A^T
-        __builtin_amdgcn_sched_barrier(0);
-    };
     // At most `steps` steps' copies of this wave in flight, no LDS read.
     auto wait_steps = [&](int steps) {
         if (NS > 4 && steps >= 4)
@@ -472,38 +453,108 @@ __global__ __launch_bounds__(128 * WGN, 1) void gemm_small_kernel(const f16* __r
     for (int t = 0; t < npro; ++t) copy_step(t, t);
     wait_steps(npro - 1 < 4 ? npro - 1 : 4);
     bare_barrier();
-    read_step(0, 0);
-    // Step t (stage buf, operands in registers q): its reads and the copies of
-    // step t + 1 have landed in every wave, so stage buf takes step t + NS and
-    // step t + 1 is read under this step's MFMAs.
     auto next = [&](int b) { return b + 1 == NS ? 0 : b + 1; };
-    int t = 0, buf = 0;
-    for (; t + 1 + NS < nk; t += 2) {
+    if constexpr (SLICED) {
+        half8v fa[2][MT], fb[2][NT];
+        auto read_slice = [&](int buf, int ks) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            wait_vm_lgkm0<(NS - 2) * kStepCopies>();
-            bare_barrier();
-            copy_step(t + u + NS, buf);
-            buf = next(buf);
-            read_step(buf, u ^ 1);
-            mfma_step(u);
-        }
-    }
-    for (; t < nk; t += 2) {
+            for (int i = 0; i < MT; ++i) fa[ks & 1][i] = *(const half8v*)(smem + buf * kABuf + ao[ks] + i * 4096);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            if (t + u < nk) {
-                const int newest = min(t + u + NS - 1, nk - 1);  // last step copied
-                wait_steps(newest - (t + u + 1));
+            for (int i = 0; i < NT; ++i) fb[ks & 1][i] = *(const half8v*)(smem + buf * kBBuf + bo[ks] + i * 4096);
+        };
+        auto mfma_slice = [&](int ks) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    acc[i][j] = mfma32(fb[ks & 1][j], fa[ks & 1][i], acc[i][j]);  // D = B A^T
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        read_slice(0, 0);
+        for (int t = 0, buf = 0; t < nk; ++t) {
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): slice 0
+#pragma unroll
+            for (int ks = 0; ks + 1 < kSlices; ++ks) {
+                read_slice(buf, ks + 1);
+                mfma_slice(ks);
+            }
+            // Once every wave has its last reads of step t and its copies of
+            // step t + 1, that step's first slice is read and stage buf refilled
+            // (reads first: 559 x 2048 x 2048 in the cache 12.9 -> 12.1 us).
+            if (t + 1 < nk) {
+                wait_steps(min(t + NS - 1, nk - 1) - (t + 1));
                 bare_barrier();
-                if (t + u + NS < nk) copy_step(t + u + NS, buf);
+                const int done = buf;
                 buf = next(buf);
-                if (t + u + 1 < nk) read_step(buf, u ^ 1);
+                read_slice(buf, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (t + NS < nk) copy_step(t + NS, done);
+            }
+            mfma_slice(kSlices - 1);
+        }
+        bare_barrier();  // every wave has its last operand reads
+    } else {
+        half8v fa[2][kSlices][MT], fb[2][kSlices][NT];
+        // The addresses step to the next stage (buf + 1, or back to 0) in place: an
+        // address made in a register the MFMAs in flight still read would wait for
+        // them (420 x 2048 x 6144: 25 against 21.5 us).
+        auto read_step = [&](int buf, int q) {
+            const int da = buf == NS - 1 ? -(NS - 1) * kABuf : kABuf;
+            const int db = buf == NS - 1 ? -(NS - 1) * kBBuf : kBBuf;
+#pragma unroll
+            for (int ks = 0; ks < kSlices; ++ks) {
+#pragma unroll
+                for (int i = 0; i < MT; ++i) fa[q][ks][i] = *(const half8v*)(smem + ao[ks] + i * 4096);
+#pragma unroll
+                for (int i = 0; i < NT; ++i) fb[q][ks][i] = *(const half8v*)(smem + bo[ks] + i * 4096);
+                ao[ks] += da;
+                bo[ks] += db;
+                asm volatile("" : "+v"(ao[ks]), "+v"(bo[ks]));
+            }
+        };
+        auto mfma_step = [&](int q) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int ks = 0; ks < kSlices; ++ks)
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) acc[i][j] = mfma32(fb[q][ks][j], fa[q][ks][i], acc[i][j]);  // D = B A^T
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        read_step(0, 0);
+        // Step t (stage buf, operands in registers q): its reads and the copies of
+        // step t + 1 have landed in every wave, so stage buf takes step t + NS and
+        // step t + 1 is read under this step's MFMAs.
+        int t = 0, buf = 0;
+        for (; t + 1 + NS < nk; t += 2) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                wait_vm_lgkm0<(NS - 2) * kStepCopies>();
+                bare_barrier();
+                copy_step(t + u + NS, buf);
+                buf = next(buf);
+                read_step(buf, u ^ 1);
                 mfma_step(u);
             }
         }
+        for (; t < nk; t += 2) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                if (t + u < nk) {
+                    const int newest = min(t + u + NS - 1, nk - 1);  // last step copied
+                    wait_steps(newest - (t + u + 1));
+                    bare_barrier();
+                    if (t + u + NS < nk) copy_step(t + u + NS, buf);
+                    buf = next(buf);
+                    if (t + u + 1 < nk) read_step(buf, u ^ 1);
+                    mfma_step(u);
+                }
+            }
+        }
     }
-    // Every wave's last operand reads returned before the last step's barrier.
+    // (Whole-step reads: every wave's last returned before the last step's barrier.)
     Epilogue<MT, NT, OUT>::run(acc, smem + wave * Epilogue<MT, NT, OUT>::kBytes, C, M, OUT == kGemmGlu ? N / 2 : N,
                                m0 + wm * WM, (n0 + wn * WN) / (OUT == kGemmGlu ? 2 : 1), lane);
 }
@@ -514,6 +565,7 @@ struct GemmCall {
     f16* C;
     int M, N, K;
     GemmOut out;
+    int64_t cus;
     hipStream_t stream;
 };
 
@@ -529,15 +581,15 @@ hipError_t launch_big(const GemmCall& c) {
     return hipGetLastError();
 }
 
-template <int BM, int BN, int NS, int WGN>
+template <int BM, int BN, int NS, int WGN, bool SLICED = false>
 hipError_t launch_small(const GemmCall& c) {
     const dim3 grid((unsigned)(((c.M + BM - 1) / BM) * (c.N / BN)));
     if (c.out == kGemmAcc)
-        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, kGemmAcc>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, SLICED, kGemmAcc>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     else if (c.out == kGemmGlu)
-        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, kGemmGlu>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, SLICED, kGemmGlu>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     else
-        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, kGemmStore>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
+        hipLaunchKernelGGL((gemm_small_kernel<BM, BN, NS, WGN, SLICED, kGemmStore>), grid, dim3(128 * WGN), 0, c.stream, c.A, c.B, c.C, c.M, c.N, c.K);
     return hipGetLastError();
 }
 
@@ -571,7 +623,12 @@ hipError_t launch_tile(const Tile& t, const GemmCall& c) {
         case 2: return launch_big<128, 256, 3, 2>(c);
         case 3: return launch_small<64, 128, 3, 2>(c);
         case 4: return launch_small<128, 64, 3, 2>(c);
-        case 5: return launch_small<64, 64, 4, 2>(c);
+        case 5: {
+            // One to 1.5 tiles a CU: slice by slice (see gemm_small_kernel).
+            const int64_t tiles = (int64_t)((c.M + 63) / 64) * (c.N / 64);
+            if (tiles > c.cus && 2 * tiles <= 3 * c.cus) return launch_small<64, 64, 4, 2, true>(c);
+            return launch_small<64, 64, 4, 2>(c);
+        }
         default: return launch_big<160, 256, 3, 1>(c);
     }
 }
@@ -612,7 +669,7 @@ hipError_t launch_gemm_f16(const f16* A, const f16* B, f16* C, int M, int N, int
                            int cus, hipStream_t stream) {
     if (!gemm_f16_fits(M, N, K)) return hipErrorInvalidValue;
     const int64_t ncu = std::max(1, cus);
-    GemmCall c{A, B, C, M, N, K, out, stream};
+    GemmCall c{A, B, C, M, N, K, out, ncu, stream};
     // QASR_GEMM_TILE = 1..7 forces that tile for all rows (the tests compare
     // them; one whose kernel needs more K steps than there are is not forced).
     const char* forced = std::getenv("QASR_GEMM_TILE");

@@ -184,3 +184,41 @@ def test_gemm_loop_edges_every_tile(gpu, m, n, k, accumulate, monkeypatch):
     ref = ref.cpu().numpy()
     bound = 0.5 * _f16_spacing(ref) + 2 * (k + 1) * 2.0 ** -24 * mag.cpu().numpy()
     assert np.all(np.abs(want.cpu().numpy().astype(np.float64) - ref) <= bound)
+
+
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 576])
+@pytest.mark.parametrize("n,per_cu,short", [(2048, 1.125, 0), (2048, 1.5, 63), (3072, 1.125, 40), (256, 1.25, 1)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_gemm_sliced_loop_keeps_bits(gpu, k, n, per_cu, short, accumulate, monkeypatch):
+    """The 64 x 64 tile with more than one and up to 1.5 tiles a CU reads its
+    operands slice by slice: K steps below, at and above its four copy stages,
+    whole and ragged last row blocks, both ends of the range; the bits are
+    those of the 128 x 64 and 64 x 128 tiles, and the fp32 bound holds."""
+    import torch
+
+    import qasr_attn
+    from gpu_helpers import say
+
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    blocks = int(per_cu * cus) // (n // 64)
+    assert cus < blocks * (n // 64) <= 1.5 * cus
+    m = 64 * blocks - short
+    g = torch.Generator(device="cuda").manual_seed(7500 + m + n + k + int(accumulate))
+    a = torch.randn((m, k), generator=g, device="cuda").to(torch.float16)
+    b = (torch.randn((n, k), generator=g, device="cuda") * 0.05).to(torch.float16)
+    c0 = torch.randn((m, n), generator=g, device="cuda").to(torch.float16)
+    outs = {}
+    for tile in (6, 5, 4):
+        monkeypatch.setenv("QASR_GEMM_TILE", str(tile))
+        say(f"gemm sliced {m}x{n}x{k} accumulate={accumulate} tile {tile}")
+        outs[tile] = c0.clone()
+        qasr_attn.gemm_f16(g_ctx(), a, b, outs[tile], accumulate=accumulate)
+    for tile in (5, 4):
+        assert torch.equal(outs[6].view(torch.int16), outs[tile].view(torch.int16)), tile
+    bt = b.float().t().contiguous()
+    ref, mag = torch.mm(a.float(), bt), torch.mm(a.float().abs(), bt.abs())
+    if accumulate:
+        ref, mag = ref + c0.float(), mag + c0.float().abs()
+    ref = ref.cpu().numpy()
+    bound = 0.5 * _f16_spacing(ref) + 2 * (k + 1) * 2.0 ** -24 * mag.cpu().numpy()
+    assert np.all(np.abs(outs[6].cpu().numpy().astype(np.float64) - ref) <= bound)
