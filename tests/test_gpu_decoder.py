@@ -468,6 +468,75 @@ def test_fused_epilogues_equal_unfused(gpu, model, batch, int8, lds, monkeypatch
     assert np.array_equal(out["fused"][1], out["unfused"][1])
 
 
+def _prefill_runs(cfg, W, rows, settings, seed, monkeypatch):
+    """(logits, KV rows) of one prompt's prefill under each of `settings`, lists
+    of (variable, value or None)."""
+    import torch
+
+    from gpu_helpers import say
+
+    hidden = _prompt(SEED_BASE + seed, rows, cfg["hs"])
+    dec = _native(cfg, W, 1, (rows + 255) // 256 * 256, max_rows=rows)
+    out = []
+    for setting in settings:
+        for name, value in setting:
+            if value is None:
+                monkeypatch.delenv(name, raising=False)
+            else:
+                monkeypatch.setenv(name, value)
+        say(f"prefill hs {cfg['hs']} inter {cfg['inter']} rows {rows}: {setting}")
+        dec.kv.tensor().zero_()
+        lg = _logits(cfg["vocab"])
+        dec.prefill(hidden, 0, logits=lg)
+        torch.cuda.synchronize()
+        out.append((lg.view(torch.int32).clone(), dec.kv.tensor()[0, :, :, :, :rows].clone().view(torch.int16)))
+    dec.close()
+    return out
+
+
+@pytest.mark.parametrize("hs,inter,rows,int8", [(1024, 3072, 300, False), (1024, 3072, 257, True),
+                                                (256, 128, 161, False), (192, 384, 1, False)])
+def test_prefill_glu_epilogue_every_tile(gpu, hs, inter, rows, int8, monkeypatch):
+    """SiLU(gate) * up in the prefill GEMM's epilogue, in every block tile (K of
+    3 steps and more, ragged last row blocks), against QASR_DECODER_FUSE=0
+    (gate|up stored, then silu_mul_kernel): logits and the next layer's K/V rows
+    bitwise."""
+    import torch
+
+    cfg = dict(CFG_0P6B, hs=hs, inter=inter, layers=2, vocab=4096)
+    W = synth_weights(cfg, SEED_BASE + 1500 + hs + rows, device="cuda")
+    if int8:
+        for key in list(W):
+            if isinstance(key, tuple) and key[1] in PROJECTIONS:
+                W[key], W[(key[0], key[1] + "_scale")] = _quantize_rows(W[key])
+    fuse, tile = "QASR_DECODER_FUSE", "QASR_GEMM_TILE"
+    settings = [[(fuse, "0"), (tile, None)]] + [[(fuse, "1"), (tile, t)] for t in (None, *"1234567")]
+    (logits, kv), *fused = _prefill_runs(cfg, W, rows, settings, 1510, monkeypatch)
+    assert torch.isfinite(logits.view(torch.float32)).all()
+    for (_, (_, t)), (lg, k) in zip(settings[1:], fused):
+        assert torch.equal(lg, logits), t
+        assert torch.equal(k, kv), t
+
+
+@pytest.mark.parametrize("model,rows", [("1.7B", 4269), ("1.7B", 1400), ("0.6B", 2900)])
+def test_prefill_glu_epilogue_two_launches(gpu, model, rows, monkeypatch):
+    """Row counts at which gate|up runs as two launches on 256 CUs (4096 rows of
+    256 x 256 tiles and 173 of 64 x 128; 960 of 192 x 256 and 440 of 128 x 256; 2560
+    of 256 x 256 and 340 of 128 x 64): logits and K/V rows as with the epilogue
+    off, bitwise."""
+    import torch
+
+    from decoder_model import CFG_1P7B
+
+    cfg = dict(CFG_1P7B if model == "1.7B" else CFG_0P6B, layers=2, vocab=4096)
+    W = synth_weights(cfg, SEED_BASE + 1520 + rows, device="cuda")
+    monkeypatch.delenv("QASR_GEMM_TILE", raising=False)
+    runs = _prefill_runs(cfg, W, rows, [[("QASR_DECODER_FUSE", f)] for f in "01"], 1530, monkeypatch)
+    assert torch.isfinite(runs[0][0].view(torch.float32)).all()
+    assert torch.equal(runs[1][0], runs[0][0])
+    assert torch.equal(runs[1][1], runs[0][1])
+
+
 @pytest.mark.parametrize("model,batch", [("0.6B", 6), ("0.6B", 8), ("1.7B", 9), ("0.6B", 12), ("1.7B", 13)])
 def test_folded_norm_row_counts(gpu, model, batch, monkeypatch):
     """The folded norm reduces only the rows there are, by one, four or all of
