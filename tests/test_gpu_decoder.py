@@ -494,7 +494,7 @@ def _prefill_runs(cfg, W, rows, settings, seed, monkeypatch):
     return out
 
 
-@pytest.mark.parametrize("hs,inter,rows,int8", [(1024, 3072, 300, False), (1024, 3072, 257, True),
+@pytest.mark.parametrize("hs,inter,rows,int8", [(1024, 3072, 300, False), (1024, 3072, 161, False), (1024, 3072, 257, True),
                                                 (256, 128, 161, False), (192, 384, 1, False)])
 def test_prefill_glu_epilogue_every_tile(gpu, hs, inter, rows, int8, monkeypatch):
     """SiLU(gate) * up in the prefill GEMM's epilogue, in every block tile (K of
