@@ -186,9 +186,9 @@ struct Epilogue {
 // tiles), 0.75 us for the 64 KB of a 256 x 256 step against 0.85 us of MFMAs,
 // so they have to run all the time.  With two stages of both operands they
 // could only be issued once a step's reads were done, and had to land before
-// the next step's: 1.4 us a step.  Three stages of A (and of B where LDS holds
-// them; two for 256 columns by 192 or 256 rows, all 160 KB) keep a third of a
-// step or more queued across the barrier: 1.1 us (4269 x 2048 x 6144 with the
+// the next step's: 1.4 us a step.  Three stages of A, and of B where LDS holds
+// them (144 KB with 128 rows, 156 KB with 160; two stages of B with 192 rows, 136 KB,
+// and 256, 160 KB), keep a third of a step or more queued across the barrier: 1.1 us (4269 x 2048 x 6144 with the
 // residual, this tile: 149 -> 118 us).
 //
 // Steps: slice ks + 1's operand reads go out one per MFMA under slice ks's
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict_
         }
     };
     using Full = std::integral_constant<int, 7>;
-    const int nk = K / kBK;  // >= 3 (gemm_big_fits)
+    const int nk = K / kBK;  // >= NB (Tile::min_steps)
 #pragma unroll
     for (int j = 0; j < ACOPY; ++j) copy_a(0, 0, j);
 #pragma unroll
@@ -581,7 +581,7 @@ hipError_t launch_big(const GemmCall& c) {
     return hipGetLastError();
 }
 
-template <int BM, int BN, int NS, int WGN, bool SLICED = false>
+template <int BM, int BN, int NS, int WGN, bool SLICED>
 hipError_t launch_small(const GemmCall& c) {
     const dim3 grid((unsigned)(((c.M + BM - 1) / BM) * (c.N / BN)));
     if (c.out == kGemmAcc)
@@ -598,15 +598,20 @@ hipError_t launch_small(const GemmCall& c) {
 // of one per CU; the small ones take step[0] alone and step[1] two to a CU
 // (in between, as the square root of the share of CUs with two), and fill in
 // behind each other, so a last part round costs little more than its share.
-// 160 x 256 was fitted at its K = 2048 and 6144 times with most CUs busy.
 // The figures are sweeps of every tile over the 1.7B and 0.6B projections at 64
 // to 4,269 rows and a 16384 x 12288 x 2048 product, weights coming from HBM.
+// 160 x 256 is charged what it takes at K = 6144 (105-110 us a busy round, 108 here),
+// which is more than it takes at K = 1024 and 2048 (21 and 37 us, 26 and 43 here):
+// with 5.5 + 0.97 a step it is also chosen for second launches of a row split, whose
+// rounds overlap the first's, and those were up to 6% slower (3400 x 6144 x 1024
+// 42.3 -> 44.9 us).  So it serves N = 2048 with a long K, one round of it for
+// 4,097 to 5,120 rows.
 struct Tile {
     int bm, bn, occ;
     float fix, step[2];
-    int min_steps;  // K steps the kernel needs
+    int min_steps;  // K steps the kernel needs: its stages of B when large (launch_tile)
 };
-const Tile kTiles[] = {{256, 256, 1, 6.5f, {1.50f, 0.0f}, 2},
+constexpr Tile kTiles[] = {{256, 256, 1, 6.5f, {1.50f, 0.0f}, 2},
                        {192, 256, 1, 6.0f, {1.10f, 0.0f}, 2},
                        {128, 256, 1, 5.5f, {0.82f, 0.0f}, 3},
                        {64, 128, 2, 4.0f, {0.40f, 0.62f}, 1},
@@ -616,20 +621,34 @@ const Tile kTiles[] = {{256, 256, 1, 6.5f, {1.50f, 0.0f}, 2},
 constexpr int kNumTiles = (int)(sizeof kTiles / sizeof kTiles[0]);
 constexpr float kSecondLaunchUs = 2.0f;
 
+// Kernel instances of kTiles[I]: the sizes come from the table, and its
+// min_steps cover the copies that a large tile issues ahead.
+template <int I, int NB, int WGM>
+hipError_t launch_big_tile(const GemmCall& c) {
+    static_assert(kTiles[I].min_steps >= NB, "steps copied ahead");
+    return launch_big<kTiles[I].bm, kTiles[I].bn, NB, WGM>(c);
+}
+
+template <int I, int NS, int WGN, bool SLICED = false>
+hipError_t launch_small_tile(const GemmCall& c) {
+    return launch_small<kTiles[I].bm, kTiles[I].bn, NS, WGN, SLICED>(c);
+}
+
 hipError_t launch_tile(const Tile& t, const GemmCall& c) {
+    static_assert(kNumTiles == 7, "one case per tile");
     switch (&t - kTiles) {
-        case 0: return launch_big<256, 256, 2, 2>(c);
-        case 1: return launch_big<192, 256, 2, 2>(c);
-        case 2: return launch_big<128, 256, 3, 2>(c);
-        case 3: return launch_small<64, 128, 3, 2>(c);
-        case 4: return launch_small<128, 64, 3, 2>(c);
+        case 0: return launch_big_tile<0, 2, 2>(c);
+        case 1: return launch_big_tile<1, 2, 2>(c);
+        case 2: return launch_big_tile<2, 3, 2>(c);
+        case 3: return launch_small_tile<3, 3, 2>(c);
+        case 4: return launch_small_tile<4, 3, 2>(c);
         case 5: {
             // One to 1.5 tiles a CU: slice by slice (see gemm_small_kernel).
             const int64_t tiles = (int64_t)((c.M + 63) / 64) * (c.N / 64);
-            if (tiles > c.cus && 2 * tiles <= 3 * c.cus) return launch_small<64, 64, 4, 2, true>(c);
-            return launch_small<64, 64, 4, 2>(c);
+            if (tiles > c.cus && 2 * tiles <= 3 * c.cus) return launch_small_tile<5, 4, 2, true>(c);
+            return launch_small_tile<5, 4, 2>(c);
         }
-        default: return launch_big<160, 256, 3, 1>(c);
+        default: return launch_big_tile<6, 3, 1>(c);
     }
 }
 
