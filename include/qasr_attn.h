@@ -245,7 +245,10 @@ typedef struct qasr_decoder qasr_decoder;
 
 /* embed_dev: [vocab][hs] (embed_tokens, also the tied lm_head);
  * final_norm_dev: [hs]; layers: num_hidden_layers entries (a host array, read
- * during the call).  Allocates the activation workspace for max_rows rows. */
+ * during the call).  Allocates the activation workspace for max_rows rows
+ * and, with int8 projections, an f16 scratch for all int8 matrices of one layer
+ * (the layer with the most: 31 MB at the 0.6B shape, 101 MB at 1.7B), which a
+ * prefill fills layer by layer. */
 int qasr_decoder_create(qasr_ctx* ctx, const qasr_decoder_cfg* cfg, const void* embed_dev,
                         const void* final_norm_dev, const qasr_layer_weights* layers,
                         qasr_decoder** out);

@@ -23,7 +23,8 @@
 // batch gives the same bits (the library's stream-K kernels split K by the
 // row count).  QASR_PREFILL_GEMM=blas sends them to rocBLAS instead (beta = 1
 // for the residual; not row invariant).  A prefill's SiLU * up is the gate|up
-// GEMM's epilogue, and its int8 projections are dequantised once per layer.  The elementwise steps are small HIP kernels below.  Nothing here allocates per
+// GEMM's epilogue, and its int8 projections are dequantised in one launch per
+// layer.  The elementwise steps are small HIP kernels below.  Nothing here allocates per
 // call: the activation workspace is sized for max_rows at creation, and
 // rocBLAS gets a fixed workspace so that a step can be captured in a graph.
 
@@ -1242,7 +1243,7 @@ struct qasr_decoder {
     rocblas_handle blas = nullptr;
     void* blas_ws = nullptr;
     hipStream_t stream = nullptr;  // of the call in progress
-    bool force_blas = false;       // QASR_DECODER_BLAS=1: every projection through rocBLAS
+    bool force_blas = false;       // QASR_DECODER_BLAS=1: no skinny kernels (gemm.hip or rocBLAS instead)
     bool fuse = true;              // QASR_DECODER_FUSE=0: no fused epilogues (same results)
     int lds_gemm = 1;              // QASR_SKINNY_LDS: 0 older kernel only, 2 LDS kernel wherever it fits
     int lds_tpw = 0, lds_groups = 0;  // QASR_SKINNY_TPW / _GROUPS: shape overrides (0 = planner)
@@ -1536,8 +1537,10 @@ SkinnyArgs skinny_args(qasr_decoder* d, SkinnyShape sh, int rows, int n_out, int
 }
 
 // y = x . W^T (+ y).  W is f16, or int8 with per-row `scale`.  Skinny shapes
-// run the MFMA skinny kernel (int8 dequantised in registers); others go to
-// rocBLAS, an int8 W first dequantised into the scratch matrix.
+// run the MFMA skinny kernel (int8 dequantised in registers); others the GEMM
+// of gemm.hip where it fits, else (or with QASR_PREFILL_GEMM=blas) rocBLAS.  A
+// prefill's int8 W has been dequantised with its layer (dequant_layer); one
+// that still has its scales is dequantised into the scratch matrix first.
 int gemm_f16(qasr_decoder* d, int rows, int n_out, int k, const void* W, const f16* x, f16* y,
              bool accumulate, const float* scale = nullptr) {
     const SkinnyShape sh = skinny_shape(d, rows, n_out, k, scale != nullptr);
