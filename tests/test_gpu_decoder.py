@@ -243,7 +243,8 @@ def test_skinny_projections_match_rocblas(gpu, model, batch, lds, monkeypatch):
     """The decode-step projections (at most 16 rows: this library's MFMA
     skinny GEMMs, split across workgroups for a long K; with
     QASR_SKINNY_LDS=2 the LDS-staged kernel takes every shape it fits, not
-    just the widest) against rocBLAS for the same steps (QASR_DECODER_BLAS=1):
+    just the widest) against rocBLAS for the same steps (QASR_DECODER_BLAS=1
+    with QASR_PREFILL_GEMM=blas, without which the prefill GEMM takes them):
     logits within rounding of each other, the same tokens wherever the top-2
     margin is clear."""
     import torch
@@ -262,6 +263,7 @@ def test_skinny_projections_match_rocblas(gpu, model, batch, lds, monkeypatch):
     out = {}
     for name, blas in (("skinny", "0"), ("rocblas", "1")):
         monkeypatch.setenv("QASR_DECODER_BLAS", blas)
+        monkeypatch.setenv("QASR_PREFILL_GEMM", "blas" if blas == "1" else "own")
         nxt = torch.empty(batch, dtype=torch.int32, device="cuda")
         lg = torch.empty((batch, cfg["vocab"]), dtype=torch.float32, device="cuda")
         say(f"{model} batch {batch}: step via {name}")
@@ -355,9 +357,9 @@ def test_int8_projections_equal_dequantized_f16(gpu, model, batch, blas, monkeyp
     """Resident int8 projections (per-row f32 scale; the reference's int8
     checkpoints, weights.rs:296-427) against the same decoder over f16
     weights dequantized on the host as f16(q * s): the decode steps (int8
-    skinny GEMM that dequantizes in registers, or rocBLAS over a dequantized
-    copy when QASR_DECODER_BLAS=1) and the prefill (dequantized copy +
-    rocBLAS) must give identical tokens and logits, bitwise."""
+    skinny GEMM that dequantizes in registers, or the prefill GEMM over a
+    dequantized copy when QASR_DECODER_BLAS=1) and the prefill (that GEMM over
+    the layer's dequantized copies) must give identical tokens and logits, bitwise."""
     import torch
 
     from decoder_model import CFG_1P7B
