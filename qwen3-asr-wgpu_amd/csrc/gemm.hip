@@ -24,13 +24,13 @@
 // of a few row blocks, so the tiles an XCD runs at one time share a few A
 // and B blocks in its L2.
 // Every output sums over K in one fixed order whatever the tile.
-// Figures here (us, one MI355X, 28 weight matrices rotated so that they come
-// from HBM, against the two-stage ping-pong and slice-by-slice loops these
-// kernels replace): 4269 x 12288 x 2048 207 -> 189, 4269 x 4096 x 2048 83 -> 68,
-// 4269 x 2048 x 2048 + residual 48 -> 41, 4269 x 2048 x 6144 + residual 138 ->
-// 107, 420 x 12288 x 2048 36.7 -> 31.5, 420 x 4096 x 2048 18.7 -> 15.8,
-// 420 x 2048 x 2048 + residual 10.9 -> 9.6, 131 x 1024 x 3072 + residual 14.5 ->
-// 11.7; weights in the memory-side cache, 420 x 2048 x 6144 + residual 25.7 -> 21.9.
+// Figures (us, one MI355X, both builds in turn, against the two-stage ping-pong
+// and slice-by-slice loops before; weight matrices rotated so that they come
+// from HBM): 4269 x 12288 x 2048 209 -> 189, 4269 x 4096 x 2048 85 -> 69, 4269 x 2048 x
+// 2048 + residual 52 -> 42, 4269 x 2048 x 6144 + residual 142 -> 106, 420 x 12288 x
+// 2048 39.5 -> 32.6, 420 x 4096 x 2048 18.6 -> 15.9, 420 x 2048 x 2048 + residual 11.4 ->
+// 11.0, 420 x 2048 x 6144 + residual 29.0 -> 28.0, 131 x 1024 x 3072 + residual 15.0 -> 14.1;
+// one matrix, in the memory-side cache: the last three 10.7 -> 9.3, 25.4 -> 21.1, 14.5 -> 11.5.
 
 #include <algorithm>
 #include <cmath>
@@ -368,7 +368,8 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const f16* __restrict_
 // LDS or memory latency is waited for: a whole step's operands are read into
 // registers under the previous step's MFMAs (one barrier per step, where a
 // read of each 16-k slice under the slice before it waited four LDS latencies:
-// 131 x 1024 x 3072 14.6 -> 11.8 us, 420 x 2048 x 6144 26.2 -> 22.4 us), and
+// 131 x 1024 x 3072 14.6 -> 11.8 us, 420 x 2048 x 6144 26.2 -> 22.4 us with the weights
+// in the memory-side cache), and
 // NS stages keep NS - 2 steps of copies in flight.
 // SLICED: each slice is read under the MFMAs of the slice before it.  Where
 // some CUs have two workgroups, the other one covers the LDS latencies and
